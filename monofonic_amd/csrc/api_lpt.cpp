@@ -138,8 +138,7 @@ int mfic_ngenic_fill(mfic_grid g, long seed) {
         ngenic_seedtable(seed, n, tab.data());
         uint32_t* dt = static_cast<uint32_t*>(ctx_scratch(g->ctx, "seedtable", n * n * sizeof(uint32_t)));
         MFIC_HIP(hipMemcpyAsync(dt, tab.data(), n * n * sizeof(uint32_t), hipMemcpyHostToDevice, g->ctx->stream));
-        grid_fill(g, 0.0);
-        ngenic_fill(g, dt);
+        ngenic_fill(g, dt);  // writes every mode
         g->space = MFIC_KSPACE;
         MFIC_HIP(hipStreamSynchronize(g->ctx->stream));
     });
@@ -401,7 +400,6 @@ int mfic_run_execute(mfic_run r, int blocking) {
         if (phi1_cubic(phi1)) {  // phi1 formed in the noise kernel's stores
             ngenic_phi1_fill(phi1, r->d_table, phi1_table(phi1, r->eh), r->coef.volfac, c.do_fixing, c.do_inversion);
         } else {
-            grid_fill(phi1, 0.0);
             ngenic_fill(phi1, r->d_table);
             phi1_from_noise(phi1, phi1, r->eh, r->coef.volfac, c.do_fixing, c.do_inversion);
         }
