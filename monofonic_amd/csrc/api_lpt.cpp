@@ -672,25 +672,20 @@ int mfic_ppt_fields(mfic_run r, double velocity_unit, mfic_grid delta, mfic_grid
         const size_t nn[3] = {n, n, n};
         const double norm = 1.0 / std::sqrt((double)n * n * n);
         // growth-scaled real-space potentials (ic_generator.cc:644-658, 809, 847)
-        struct Buf {
-            void* p = nullptr;
-            ~Buf() {
-                if (p) (void)hipFree(p);
-            }
-        } ph1, ph2, psi, grad;
-        const size_t greal = n * n * (n + 2) * es;
-        ph1.p = dmalloc(greal, "PPT phi");
-        if (c.lpt_order >= 2) ph2.p = dmalloc(greal, "PPT phi2");
-        psi.p = dmalloc(n * n * n * 2 * es, "PPT psi");
-        grad.p = dmalloc(n * n * n * 2 * es, "PPT grad psi");
-        MFIC_HIP(hipMemcpyAsync(ph1.p, r->pot[0]->d, greal, hipMemcpyDeviceToDevice, r->ctx->stream));
-        if (ph2.p) MFIC_HIP(hipMemcpyAsync(ph2.p, r->pot[1]->d, greal, hipMemcpyDeviceToDevice, r->ctx->stream));
+        // and psi, in the workspace of the LPT sources (a run of order 2 or 3
+        // has one that is large enough)
+        const size_t greal = n * n * (n + 2) * es, slot = (greal + 255) / 256 * 256;
+        char* ws = static_cast<char*>(ctx_scratch(r->ctx, "fused_in", 2 * slot + n * n * n * 2 * es));
+        void* ph1 = ws;
+        void* ph2 = c.lpt_order >= 2 ? ws + slot : nullptr;
+        MFIC_HIP(hipMemcpyAsync(ph1, r->pot[0]->d, greal, hipMemcpyDeviceToDevice, r->ctx->stream));
+        if (ph2) MFIC_HIP(hipMemcpyAsync(ph2, r->pot[1]->d, greal, hipMemcpyDeviceToDevice, r->ctx->stream));
         if (c.prec == MFIC_F64) {
-            fft_c2r<double>(r->ctx, (double*)ph1.p, nn, norm * r->coef.g1);
-            if (ph2.p) fft_c2r<double>(r->ctx, (double*)ph2.p, nn, norm * r->coef.g2);
+            fft_c2r<double>(r->ctx, (double*)ph1, nn, norm * r->coef.g1);
+            if (ph2) fft_c2r<double>(r->ctx, (double*)ph2, nn, norm * r->coef.g2);
         } else {
-            fft_c2r<float>(r->ctx, (float*)ph1.p, nn, norm * r->coef.g1);
-            if (ph2.p) fft_c2r<float>(r->ctx, (float*)ph2.p, nn, norm * r->coef.g2);
+            fft_c2r<float>(r->ctx, (float*)ph1, nn, norm * r->coef.g1);
+            if (ph2) fft_c2r<float>(r->ctx, (float*)ph2, nn, norm * r->coef.g2);
         }
         PptInput in;
         in.n = (int)n;
@@ -698,10 +693,9 @@ int mfic_ppt_fields(mfic_run r, double velocity_unit, mfic_grid delta, mfic_grid
         in.L = c.L;
         in.Dplus0 = r->coef.Dplus0;
         in.vunit = r->coef.Dplus0 * r->coef.vfac / c.L * velocity_unit;
-        in.phi_r = ph1.p;
-        in.phi2_r = ph2.p;
-        in.psi = psi.p;
-        in.grad = grad.p;
+        in.phi_r = ph1;
+        in.phi2_r = ph2;
+        in.psi = ws + 2 * slot;
         void* vel[3] = {vx->d, vy->d, vz->d};
         ppt_fields(r->ctx, c.prec, in, delta->d, vel, hbar);
         MFIC_HIP(hipStreamSynchronize(r->ctx->stream));

@@ -14,7 +14,7 @@ struct PptInput {
     double L = 0, Dplus0 = 0;
     double vunit = 0;                          // D+ vfac / L * velocity_unit
     const void *phi_r = nullptr, *phi2_r = nullptr;  // growth-scaled, real [n][n][n+2]
-    void *psi = nullptr, *grad = nullptr;      // [n][n][n] complex work arrays
+    void* psi = nullptr;                       // [n][n][n] complex work array
 };
 // delta and vel[0..2]: real [n][n][n+2] grids of the input precision
 void ppt_fields(mfic_ctx ctx, int prec, const PptInput& in, void* delta, void* vel[3], double* hbar);
