@@ -420,7 +420,7 @@ int mfic_fft_set_plan(mfic_ctx ctx, int length, int pass, int prec, int variant)
     return guard([&] {
         check_plan_key(ctx, length, pass, prec);
         const auto key = std::make_tuple(length, pass, prec);
-        if (variant <= 0) { ctx->plans.erase(key); return; }
+        if (variant < 0) { ctx->plans.erase(key); return; }
         if (pass == MFIC_PASS_FUSED_ROWS) {  // two forms at every padded length
             MFIC_CHECK(variant < 2, MFIC_ERR_ARG, "the fused row passes have two forms");
             ctx->plans[key] = variant;

@@ -149,13 +149,11 @@ double autotune_config(mfic_ctx ctx, const mfic_ic_config& cfg, const mfic_cosmo
                 float best = cur;
                 for (int v = 0; v < k.count; ++v) {
                     if (v == had) continue;
-                    if (v) ctx->plans[key] = v;
-                    else ctx->plans.erase(key);
+                    ctx->plans[key] = v;
                     const float t = time_once();
                     if (t < best) { best = t; best_v = v; }
                 }
-                if (best_v) ctx->plans[key] = best_v;
-                else ctx->plans.erase(key);
+                ctx->plans[key] = best_v;
                 cur = best;
             }
         };

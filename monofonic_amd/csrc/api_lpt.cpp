@@ -19,9 +19,9 @@
 
 struct mfic_conv_s {
     std::unique_ptr<mfic::ConvCore> core;
-    void *kbuf = nullptr, *r1 = nullptr, *r2 = nullptr, *fbuf = nullptr;
+    void *kbuf = nullptr, *fbuf = nullptr;
     ~mfic_conv_s() {
-        for (void* p : {kbuf, r1, r2, fbuf})
+        for (void* p : {kbuf, fbuf})
             if (p) (void)hipFree(p);
     }
 };
@@ -97,6 +97,37 @@ static void compute_coefs(const mfic_cosmo_params& p, size_t n, double L, int or
     k->vfac3 = 3 * k->vfac;
 }
 
+// the six component grids through the strided c2r passes, the same with a
+// shifted pair of sub-lattices (pair pr: grids 12 pr + q and 12 pr + 6 + q
+// from grid q), and through the whole c2r transform
+template <typename T> static void cols_of(mfic_ctx ctx, mfic_grid* g, const size_t n[3]) {
+    T* d[6];
+    for (int q = 0; q < 6; ++q) d[q] = static_cast<T*>(g[q]->d);
+    fft_c2r_cols<T>(ctx, d, 6, n);
+}
+template <typename T>
+static void shifted_cols_of(mfic_ctx ctx, mfic_grid* g, int pr, const size_t n[3], const int* wa, const int* wb) {
+    T *src[6], *a[6], *b[6];
+    for (int q = 0; q < 6; ++q) {
+        src[q] = static_cast<T*>(g[q]->d);
+        a[q] = static_cast<T*>(g[q + 12 * pr]->d);
+        b[q] = static_cast<T*>(g[q + 12 * pr + 6]->d);
+    }
+    fft_c2r_cols_shift<T>(ctx, src, a, b, 6, n, wa, wb);
+}
+template <typename T> static void fields_of(mfic_ctx ctx, mfic_grid* g, const size_t n[3], double norm) {
+    T* d[6];
+    for (int q = 0; q < 6; ++q) d[q] = static_cast<T*>(g[q]->d);
+    fft_c2r<T>(ctx, d, d, 6, n, norm);
+}
+
+// a k-space grid transformed into another buffer
+template <typename T> static void real_of(mfic_ctx ctx, mfic_grid g, void* out, const size_t n[3], double scale) {
+    const T* src = static_cast<const T*>(g->d);
+    T* dst = static_cast<T*>(out);
+    fft_c2r<T>(ctx, &src, &dst, 1, n, scale);
+}
+
 static void component_coefs(const mfic_lpt_coef& k, int comp, double cf[4]) {
     if (comp < 3) {
         cf[0] = k.g1; cf[1] = k.g2; cf[2] = k.g3; cf[3] = k.g3c;
@@ -150,9 +181,7 @@ int mfic_conv_create(mfic_ctx ctx, const size_t n[3], const double L[3], int pre
         auto c = std::make_unique<mfic_conv_s>();
         c->core = std::make_unique<ConvCore>(ctx, n, L, prec);
         const size_t es = c->core->esize();
-        c->kbuf = dmalloc(c->core->kbuf_reals() * es, "convolver padded k buffer");
-        c->r1 = dmalloc(c->core->real_reals() * es, "convolver padded real buffer");
-        c->r2 = dmalloc(c->core->real_reals() * es, "convolver padded real buffer");
+        c->kbuf = dmalloc(3 * c->core->kbuf_reals() * es, "convolver padded k buffers");
         c->fbuf = dmalloc(c->core->grid_reals() * es, "convolver N-grid buffer");
         ++ctx->children;
         *out = c.release();
@@ -183,7 +212,7 @@ int mfic_conv_convolve2(mfic_conv c, const mfic_operand* a, const mfic_operand* 
         MFIC_CHECK(op >= MFIC_OP_ASSIGN && op <= MFIC_OP_MADD, MFIC_ERR_ARG, "bad output operator");
         const OperandDesc da = to_desc(a), db = to_desc(b);
         MFIC_CHECK(a->f->prec == c->core->prec && b->f->prec == c->core->prec, MFIC_ERR_ARG, "precision mismatch");
-        c->core->convolve2(da, db, out->d, op, coef, c->kbuf, c->r1, c->r2);
+        c->core->convolve2(da, db, out->d, op, coef, c->kbuf);
         out->space = MFIC_KSPACE;
     });
 }
@@ -194,7 +223,7 @@ int mfic_conv_convolve3(mfic_conv c, const mfic_operand* a, const mfic_operand* 
         conv_check_out(c, out);
         MFIC_CHECK(op >= MFIC_OP_ASSIGN && op <= MFIC_OP_MADD, MFIC_ERR_ARG, "bad output operator");
         const OperandDesc da = to_desc(a), db = to_desc(b), dc = to_desc(cc);
-        c->core->convolve3(da, db, dc, out->d, op, coef, c->kbuf, c->r1, c->r2, c->fbuf);
+        c->core->convolve3(da, db, dc, out->d, op, coef, c->kbuf, c->fbuf);
         out->space = MFIC_KSPACE;
     });
 }
@@ -427,42 +456,39 @@ int mfic_run_execute(mfic_run r, int blocking) {
             static const int SUB[3][4][3] = {{{0, 0, 0}},
                                              {{0, 0, 0}, {1, 1, 1}},
                                              {{0, 0, 0}, {0, 1, 1}, {1, 0, 1}, {1, 1, 0}}};
-            const size_t cbytes = og[0]->bytes();
-            // strided passes per component, every sub-lattice's phase formed
-            // in the axis-0 pass from one load per output pair, then the
+            // strided passes of the six components, every sub-lattice's phase
+            // formed in the axis-0 pass from one load per output pair, then the
             // contiguous pass fused with the readout of the three components
             // of each sub-lattice; gw = global offset of the species' lattice
             auto species = [&](const int gw[3], double* dpos, double* dvel) {
                 const bool global = gw[0] || gw[1] || gw[2];
-                for (int q = 0; q < 6; ++q) {
-                    if (nsub == 1 && !global) {
-                        if (c.prec == MFIC_F64) fft_c2r_cols<double>(r->ctx, (double*)og[q]->d, nn);
-                        else fft_c2r_cols<float>(r->ctx, (float*)og[q]->d, nn);
-                        continue;
-                    }
+                if (nsub == 1 && !global) {
+                    if (c.prec == MFIC_F64) cols_of<double>(r->ctx, og, nn);
+                    else cols_of<float>(r->ctx, og, nn);
+                } else {
                     int w[4][3];
                     for (int s = 0; s < 4; ++s)
                         for (int a = 0; a < 3; ++a) w[s][a] = gw[a] + SUB[c.lattice][s < nsub ? s : 0][a];
-                    if (nsub == 4)  // fcc: the second pair of sub-lattices from a copy of the component
-                        MFIC_HIP(hipMemcpyAsync(og[q + 12]->d, og[q]->d, cbytes, hipMemcpyDeviceToDevice, r->ctx->stream));
-                    for (int pr = 0; pr < (nsub == 4 ? 2 : 1); ++pr) {
-                        void* a = og[q + 12 * pr]->d;
-                        void* b = og[q + 12 * pr + 6]->d;
-                        const int* wa = (pr == 0 && !global && nsub == 2) ? nullptr : w[2 * pr];
-                        const int* wb = (pr == 0 && !global && nsub == 2) ? nullptr : w[2 * pr + 1];
-                        if (c.prec == MFIC_F64) fft_c2r_cols_shift<double>(r->ctx, (double*)a, (double*)b, nn, wa, wb);
-                        else fft_c2r_cols_shift<float>(r->ctx, (float*)a, (float*)b, nn, wa, wb);
+                    // fcc: the second pair of sub-lattices first, out of place,
+                    // then the first pair over the components themselves
+                    for (int pr = nsub == 4 ? 1 : 0; pr >= 0; --pr) {
+                        const bool plain = pr == 0 && !global && nsub == 2;
+                        const int* wa = plain ? nullptr : w[2 * pr];
+                        const int* wb = plain ? nullptr : w[2 * pr + 1];
+                        if (c.prec == MFIC_F64) shifted_cols_of<double>(r->ctx, og, pr, nn, wa, wb);
+                        else shifted_cols_of<float>(r->ctx, og, pr, nn, wa, wb);
                     }
                 }
-                for (int s = 0; s < nsub; ++s) {
-                    const void* fp[3] = {og[6 * s]->d, og[6 * s + 1]->d, og[6 * s + 2]->d};
-                    const void* fv[3] = {og[6 * s + 3]->d, og[6 * s + 4]->d, og[6 * s + 5]->d};
-                    const size_t pbase = (size_t)s * c.n * c.n * c.n;
-                    double sh[3];
-                    for (int a = 0; a < 3; ++a) sh[a] = 0.5 * (gw[a] + SUB[c.lattice][s][a]);
-                    rows_c2r_particles(r->ctx, c.prec, fp, (int)c.n, 1, c.lunit, sh, pbase, dpos);
-                    rows_c2r_particles(r->ctx, c.prec, fv, (int)c.n, 0, 0.0, sh, pbase, dvel);
-                }
+                ParticleRows pr[8];
+                for (int s = 0; s < nsub; ++s)
+                    for (int v = 0; v < 2; ++v) {
+                        ParticleRows& p = pr[2 * s + v];
+                        for (int d = 0; d < 3; ++d) p.f[d] = og[6 * s + 3 * v + d]->d;
+                        p.is_pos = v == 0;
+                        p.dst = (v == 0 ? dpos : dvel) + 3 * (size_t)s * c.n * c.n * c.n;
+                        for (int a = 0; a < 3; ++a) p.shift[a] = 0.5 * (gw[a] + SUB[c.lattice][s][a]);
+                    }
+                rows_c2r_particles(r->ctx, c.prec, pr, 2 * nsub, (int)c.n, c.lunit);
             };
             const int zero[3] = {0, 0, 0};
             species(zero, r->d_pos, r->d_vel);
@@ -481,11 +507,9 @@ int mfic_run_execute(mfic_run r, int blocking) {
                 species(gw, r->d_pos_b, r->d_vel_b);
             }
         } else {
-            for (int q = 0; q < 6; ++q) {
-                if (c.prec == MFIC_F64) fft_c2r<double>(r->ctx, (double*)og[q]->d, nn, norm);
-                else fft_c2r<float>(r->ctx, (float*)og[q]->d, nn, norm);
-                og[q]->space = MFIC_RSPACE;
-            }
+            if (c.prec == MFIC_F64) fields_of<double>(r->ctx, og, nn, norm);
+            else fields_of<float>(r->ctx, og, nn, norm);
+            for (int q = 0; q < 6; ++q) og[q]->space = MFIC_RSPACE;
         }
         if (blocking) MFIC_HIP(hipStreamSynchronize(r->ctx->stream));
     });
@@ -678,14 +702,12 @@ int mfic_ppt_fields(mfic_run r, double velocity_unit, mfic_grid delta, mfic_grid
         char* ws = static_cast<char*>(ctx_scratch(r->ctx, "fused_in", 2 * slot + n * n * n * 2 * es));
         void* ph1 = ws;
         void* ph2 = c.lpt_order >= 2 ? ws + slot : nullptr;
-        MFIC_HIP(hipMemcpyAsync(ph1, r->pot[0]->d, greal, hipMemcpyDeviceToDevice, r->ctx->stream));
-        if (ph2) MFIC_HIP(hipMemcpyAsync(ph2, r->pot[1]->d, greal, hipMemcpyDeviceToDevice, r->ctx->stream));
-        if (c.prec == MFIC_F64) {
-            fft_c2r<double>(r->ctx, (double*)ph1, nn, norm * r->coef.g1);
-            if (ph2) fft_c2r<double>(r->ctx, (double*)ph2, nn, norm * r->coef.g2);
-        } else {
-            fft_c2r<float>(r->ctx, (float*)ph1, nn, norm * r->coef.g1);
-            if (ph2) fft_c2r<float>(r->ctx, (float*)ph2, nn, norm * r->coef.g2);
+        // growth-scaled real-space potentials (ic_generator.cc:644-658, 809, 847)
+        if (c.prec == MFIC_F64) real_of<double>(r->ctx, r->pot[0], ph1, nn, norm * r->coef.g1);
+        else real_of<float>(r->ctx, r->pot[0], ph1, nn, norm * r->coef.g1);
+        if (ph2) {
+            if (c.prec == MFIC_F64) real_of<double>(r->ctx, r->pot[1], ph2, nn, norm * r->coef.g2);
+            else real_of<float>(r->ctx, r->pot[1], ph2, nn, norm * r->coef.g2);
         }
         PptInput in;
         in.n = (int)n;

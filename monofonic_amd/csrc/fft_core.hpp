@@ -413,18 +413,15 @@ __device__ __forceinline__ void fft_regs(cx<T>* v, int q, cx<T>* lds, MAP m, con
     if constexpr (S > 3) fft_stage<T, L, 3 % S, FWD, MAP, SYNC, SPLIT, V>(v, q, lds, m, tw);
 }
 
-// Pencil passes (TK neighbouring columns per workgroup) with one transform
-// exchange real and imaginary parts separately (SPLIT): with 16-column
-// tiles of 768-point pencils this lets three workgroups share a CU instead
-// of one.  Passes with two transforms per pencil (filters) keep complex
-// exchanges, whose barriers are half as many.
-template <typename T, bool SPLIT> constexpr size_t pencil_lds_elem() { return SPLIT ? sizeof(T) : sizeof(cx<T>); }
+// Pencil passes (TK neighbouring columns per workgroup) exchange real and
+// imaginary parts separately (SPLIT): with 16-column tiles of 768-point
+// pencils this lets three workgroups share a CU instead of one.
 // default LDS budget of a pencil tile: 128-byte row segments per pencil
 // position (16 complex FP32 columns) at 768 points, 32 at 512
-template <bool SPLIT> constexpr size_t pencil_lds_cap() { return SPLIT ? 69632 : 139264; }
-template <typename T, int L, bool FWD, bool SPLIT = true, int V = 0>
+constexpr size_t PENCIL_LDS_CAP = 69632;
+template <typename T, int L, bool FWD, int V = 0>
 __device__ __forceinline__ void fft_pencil(cx<T>* v, int q, cx<T>* lds, LdsMap m, const cx<T>* __restrict__ tw) {
-    fft_regs<T, L, FWD, LdsMap, BlockSync, SPLIT, V>(v, q, lds, m, tw);
+    fft_regs<T, L, FWD, LdsMap, BlockSync, true, V>(v, q, lds, m, tw);
 }
 
 // Two transforms of the same length and positions (registers v and w) in

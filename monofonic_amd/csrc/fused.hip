@@ -16,7 +16,9 @@
 // separate the three phases.  Two forms: one half-length transform per row
 // (k_rows_fused) or two rows per full-length complex transform
 // (k_rows_fused_pair, the default), chosen per length and precision at run
-// time.
+// time.  The products of the convolver and of the 2LPT adjoint use the second.
+//
+// This file is compiled once per precision (MFIC_UNIT 32 or 64).
 #include <cmath>
 
 #include "fft_core.hpp"
@@ -25,10 +27,16 @@
 
 namespace mfic {
 
+// Products at one real point: NF fields in, NOF products out.  The paired form
+// takes ROWS padded rows together.  With two, a pair is two neighbouring rows
+// of one field: an odd number of inputs or outputs pairs up, and fields of
+// different size (the operands of a convolver call, the adjoint's lambda)
+// keep their own rounding, where a shared transform would give the smaller
+// one the larger one's.
 // Hessian component order in every source: xx yy zz xy xz yz
 // 2LPT source (ic_generator.cc:536-541)
 struct ProdSrc2 {
-    static constexpr int NI = 6, NO = 1, IPG = 1, WAVES = 3;
+    static constexpr int NF = 6, NOF = 1, ROWS = 2, WAVES = 3;
     static constexpr bool OUT32 = false;
     __device__ static __forceinline__ void eval(const double* h, double* o) {
         o[0] = h[0] * (h[1] + h[2]) + h[1] * h[2] - h[3] * h[3] - h[4] * h[4] - h[5] * h[5];
@@ -38,7 +46,7 @@ struct ProdSrc2 {
 // factor: Qzz = xx yy - xy^2, Qyz = xy xz, Qxx = yz^2, Qyy = xz^2
 // (ic_generator.cc:581-585)
 struct ProdSrc2Q {
-    static constexpr int NI = 6, NO = 5, IPG = 1, WAVES = 3;
+    static constexpr int NF = 6, NOF = 5, ROWS = 2, WAVES = 3;
     static constexpr bool OUT32 = false;
     __device__ static __forceinline__ void eval(const double* h, double* o) {
         ProdSrc2::eval(h, o);
@@ -52,11 +60,10 @@ struct ProdSrc2Q {
 // ic_generator.cc:581-609) and A3 (ic_generator.cc:614-627).  Inputs: phi1
 // Hessians a[0..5], phi2 Hessians b[6..11], Qzz Qyz Qxx Qyy [12..15]
 struct ProdSrc3 {
-    // two inputs per lane group: 4-wave workgroups; registers for two waves
-    // per SIMD (no spills), i.e. two workgroups per CU
-    static constexpr int NI = 16, NO = 4, IPG = 1, WAVES = 2;
-    // the four output transforms on 32 threads each (two waves) instead of
-    // 16 (one wave): the output phase was a third of the pass
+    // registers for two waves per SIMD (no spills), i.e. two workgroups per CU
+    static constexpr int NF = 16, NOF = 4, ROWS = 1, WAVES = 2;
+    // half-length form: the four output transforms on 32 threads each (two
+    // waves) instead of 16 (one wave): the output phase was a third of the pass
     static constexpr bool OUT32 = true;
     __device__ static __forceinline__ void eval(const double* h, double* o) {
         const double* a = h;
@@ -73,6 +80,29 @@ struct ProdSrc3 {
         o[3] = b[4] * a[5] - b[5] * a[4] + a[3] * (b[0] - b[1]) - b[3] * (a[0] - a[1]);
     }
 };
+// convolver products: two operands, or one with itself
+struct ProdMul {
+    static constexpr int NF = 2, NOF = 1, ROWS = 2, WAVES = 3;
+    __device__ static __forceinline__ void eval(const double* h, double* o) { o[0] = h[0] * h[1]; }
+};
+struct ProdSquare {
+    static constexpr int NF = 1, NOF = 1, ROWS = 2, WAVES = 3;
+    __device__ static __forceinline__ void eval(const double* h, double* o) { o[0] = h[0] * h[0]; }
+};
+// adjoint of the 2LPT source: phi1 Hessians a[0..5] and lambda [6] -> lambda
+// times the derivative of the source with respect to each Hessian
+struct ProdAdjoint2 {
+    static constexpr int NF = 7, NOF = 6, ROWS = 2, WAVES = 3;
+    __device__ static __forceinline__ void eval(const double* a, double* o) {
+        const double l = a[6];
+        o[0] = l * (a[1] + a[2]);
+        o[1] = l * (a[0] + a[2]);
+        o[2] = l * (a[0] + a[1]);
+        o[3] = -2.0 * (l * a[3]);
+        o[4] = -2.0 * (l * a[4]);
+        o[5] = -2.0 * (l * a[5]);
+    }
+};
 
 template <int M, int NI> constexpr int fused_rows_per_block() {
     constexpr int tpr = NI * lane_slot<Plan<M>::P>();
@@ -81,16 +111,15 @@ template <int M, int NI> constexpr int fused_rows_per_block() {
 
 // FP32: at least PR::WAVES waves per SIMD (register budget 512 / WAVES)
 template <typename T, int M, class PR>
-__global__ void __launch_bounds__((fused_rows_per_block<M, PR::NI / PR::IPG>() * (PR::NI / PR::IPG) * lane_slot<Plan<M>::P>()))
+__global__ void __launch_bounds__((fused_rows_per_block<M, PR::NF>() * PR::NF * lane_slot<Plan<M>::P>()))
 __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? PR::WAVES : 1, 8)))
 k_rows_fused(const cx<T>* __restrict__ in, long istride, cx<T>* __restrict__ out, long ostride, int kc, long nrows,
              T scale, const cx<T>* __restrict__ tw, const cx<T>* __restrict__ tw2) {
-    constexpr int NI = PR::NI, NO = PR::NO, IPG = PR::IPG, NG = NI / IPG;
+    constexpr int NI = PR::NF, NO = PR::NOF, NG = NI;
     constexpr int E = Plan<M>::E, P = Plan<M>::P, SL = lane_slot<P>();
     constexpr int RP = row_lds_pitch<M>(), RB = fused_rows_per_block<M, NG>(), TPR = NG * SL;
     constexpr int NPOS = (M + TPR - 1) / TPR;
     static_assert(P <= 64 && 64 % SL == 0, "a transform must fit in one wavefront");
-    static_assert(NI % IPG == 0, "inputs per group must divide the inputs");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
     const int tr = threadIdx.x % TPR, rb = threadIdx.x / TPR;
@@ -100,51 +129,39 @@ k_rows_fused(const cx<T>* __restrict__ in, long istride, cx<T>* __restrict__ out
     const bool active = row < nrows;
     const cx<T>* uw = tw + plan_tw_size<M>();
 
-    // 1. c2r of inputs g*IPG .. g*IPG+IPG-1: half-spectrum rows (kz < kc, kz = 0
-    // and the padded Nyquist real) -> M complex = 2M real values, each kept in
-    // its input's region; every row load is issued before the first transform
+    // 1. c2r of input g: half-spectrum row (kz < kc, kz = 0 and the padded
+    // Nyquist real) -> M complex = 2M real values, kept in its input's region
     if (lane) {
         // kc = N/2 + 1 with N = 4M/3: positions below KC carry data, the rest
         // of the padded row is the zero band
         constexpr int KC = 2 * M / 3 + 1;
-        cx<T> raw[IPG][E];
+        const cx<T>* src = in + g * istride + (active ? row : 0) * (long)KC;
+        const LdsRowMap lm{(rb * NI + g) * RP};
 #pragma unroll
-        for (int t = 0; t < IPG; ++t) {
-            const cx<T>* src = in + (g * IPG + t) * istride + (active ? row : 0) * (long)KC;
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const int k = q + P * e;
-                if (P * e + P <= KC) raw[t][e] = src[k];
-                else if (P * e < KC) raw[t][e] = k < KC ? src[k] : cx<T>{0, 0};
-                else raw[t][e] = cx<T>{0, 0};
-            }
+        for (int e = 0; e < E; ++e) {
+            const int k = q + P * e;
+            cx<T> x = cx<T>{0, 0};
+            if (P * e + P <= KC) x = src[k];
+            else if (P * e < KC) x = k < KC ? src[k] : cx<T>{0, 0};
+            if (k == 0) x.y = 0;
+            lds[lm.at(k)] = x;
         }
+        if (q == 0) lds[lm.at(M)] = cx<T>{0, 0};
+        WaveSync::sync();
+        cx<T> v[E];
 #pragma unroll
-        for (int t = 0; t < IPG; ++t) {
-            const LdsRowMap lm{(rb * NI + g * IPG + t) * RP};
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                cx<T> x = raw[t][e];
-                if (q + P * e == 0) x.y = 0;
-                lds[lm.at(q + P * e)] = x;
-            }
-            if (q == 0) lds[lm.at(M)] = cx<T>{0, 0};
-            WaveSync::sync();
-            cx<T> v[E];
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const int k = q + P * e;
-                const cx<T> xk = lds[lm.at(k)], xm = lds[lm.at(M - k)];
-                const cx<T> A = {xk.x + xm.x, xk.y - xm.y};
-                const cx<T> D = {xk.x - xm.x, xk.y + xm.y};
-                const cx<T> B = cmulc(D, uw[k]);
-                v[e] = cx<T>{A.x - B.y, A.y + B.x};
-            }
-            WaveSync::sync();
-            fft_regs_row<T, M, false, WaveSync>(v, q, lds, lm.base, tw);
-#pragma unroll
-            for (int e = 0; e < E; ++e) lds[lm.at(q + P * e)] = cscale(v[e], scale);
+        for (int e = 0; e < E; ++e) {
+            const int k = q + P * e;
+            const cx<T> xk = lds[lm.at(k)], xm = lds[lm.at(M - k)];
+            const cx<T> A = {xk.x + xm.x, xk.y - xm.y};
+            const cx<T> D = {xk.x - xm.x, xk.y + xm.y};
+            const cx<T> B = cmulc(D, uw[k]);
+            v[e] = cx<T>{A.x - B.y, A.y + B.x};
         }
+        WaveSync::sync();
+        fft_regs_row<T, M, false, WaveSync>(v, q, lds, lm.base, tw);
+#pragma unroll
+        for (int e = 0; e < E; ++e) lds[lm.at(q + P * e)] = cscale(v[e], scale);
     }
     __syncthreads();
 
@@ -251,14 +268,16 @@ template <typename T, int L2, int GI> constexpr int pair_rows_per_block() {
     constexpr int tpr = GI * lane_slot<Plan<L2, pair_in_variant<T, L2>()>::P>();
     return tpr >= 256 ? 1 : (256 / tpr > 8 ? 8 : 256 / tpr);
 }
+template <class PR> constexpr int pair_inputs() { return PR::NF * PR::ROWS / 2; }
+template <class PR> constexpr int pair_outputs() { return (PR::NOF * PR::ROWS + 1) / 2; }
 template <typename T, int L2, class PR> constexpr int pair_block_threads() {
-    constexpr int GI = PR::NI / 2;
+    constexpr int GI = pair_inputs<PR>();
     return pair_rows_per_block<T, L2, GI>() * GI * lane_slot<Plan<L2, pair_in_variant<T, L2>()>::P>();
 }
 // output transforms on 64 lanes (plan pair_out_plan) where every output
 // pair of the block gets a wavefront, else on the input transforms' lanes
 template <typename T, int L2, class PR> constexpr int pair_out_variant() {
-    constexpr int GO = (PR::NO + 1) / 2, RB = pair_rows_per_block<T, L2, PR::NI / 2>();
+    constexpr int GO = pair_outputs<PR>(), RB = pair_rows_per_block<T, L2, pair_inputs<PR>()>();
     constexpr int VO = pair_out_plan<L2>();
     return VO != 0 && RB * GO * lane_slot<Plan<L2, VO>::P>() <= pair_block_threads<T, L2, PR>() ? VO
                                                                                                : pair_in_variant<T, L2>();
@@ -274,7 +293,8 @@ __global__ void __launch_bounds__((pair_block_threads<T, L2, PR>()))
 __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? PR::WAVES : 1, 8)))
 k_rows_fused_pair(const cx<T>* __restrict__ in, long istride, cx<T>* __restrict__ out, long ostride, long nrows,
                   double scale2, const cx<T>* __restrict__ tw, const cx<T>* __restrict__ two) {
-    constexpr int NI = PR::NI, NO = PR::NO, GI = NI / 2, GO = (NO + 1) / 2;
+    constexpr int NF = PR::NF, NOF = PR::NOF, ROWS = PR::ROWS, NI = NF * ROWS, NO = NOF * ROWS;
+    constexpr int GI = pair_inputs<PR>(), GO = pair_outputs<PR>();
     constexpr int VI = pair_in_variant<T, L2>(), VO = pair_out_variant<T, L2, PR>();
     constexpr int E = Plan<L2, VI>::E, P = Plan<L2, VI>::P, SL = lane_slot<P>();
     constexpr int EO = Plan<L2, VO>::E, PO = Plan<L2, VO>::P, SLO = lane_slot<PO>();
@@ -287,16 +307,18 @@ k_rows_fused_pair(const cx<T>* __restrict__ in, long istride, cx<T>* __restrict_
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
     const int tr = threadIdx.x % TPR, rb = threadIdx.x / TPR;
     const int g = tr / SL, q = tr % SL;
+    // groups of ROWS consecutive rows; input i of a group is field i / ROWS
+    // of its row i % ROWS, output o product o / ROWS of its row o % ROWS
     const long tile = xcd_tile(blockIdx.x, gridDim.x);
-    const long row = tile * RB + rb;
-    const bool active = row < nrows;
+    const long group = tile * RB + rb, ngroups = nrows / ROWS;
 
     // 1. inverse transform of input pair g: all compact-row loads first, the
     // zero band (N/2 < k < L2 - N/2) never loaded
     if (q < P) {
-        const long r0 = (active ? row : 0) * (long)KC;
-        const cx<T>* s0 = in + (2 * g) * istride + r0;
-        const cx<T>* s1 = in + (2 * g + 1) * istride + r0;
+        const long r0 = (group < ngroups ? group : 0) * (long)(ROWS * KC);
+        const int i0 = 2 * g, i1 = 2 * g + 1;
+        const cx<T>* s0 = in + (i0 / ROWS) * istride + r0 + (i0 % ROWS) * KC;
+        const cx<T>* s1 = in + (i1 / ROWS) * istride + r0 + (i1 % ROWS) * KC;
         cx<T> a[E], b[E];
 #pragma unroll
         for (int e = 0; e < E; ++e) {
@@ -350,7 +372,15 @@ k_rows_fused_pair(const cx<T>* __restrict__ in, long istride, cx<T>* __restrict_
                 h[2 * p] = (double)z.x;
                 h[2 * p + 1] = (double)z.y;
             }
-            PR::eval(h, o);
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                double hr[NF], orow[NOF];
+#pragma unroll
+                for (int f = 0; f < NF; ++f) hr[f] = h[f * ROWS + r];
+                PR::eval(hr, orow);
+#pragma unroll
+                for (int f = 0; f < NOF; ++f) o[f * ROWS + r] = orow[f];
+            }
 #pragma unroll
             for (int p = 0; p < GO; ++p) {
                 const T lo = (T)(o[2 * p] * scale2);
@@ -378,10 +408,11 @@ k_rows_fused_pair(const cx<T>* __restrict__ in, long istride, cx<T>* __restrict_
             for (int e = 0; e < EO; ++e)
                 if (PO * e + PO > L2 - KC + 1) lds[base + qo + PO * e] = v[e];
             WaveSync::sync();
-            const long rowo = tile * RB + rbo;
-            if (rowo < nrows) {
-                cx<T>* d0 = out + (2 * p) * ostride + rowo * (long)KC;
-                cx<T>* d1 = out + (2 * p + 1 < NO ? 2 * p + 1 : 2 * p) * ostride + rowo * (long)KC;
+            const long groupo = tile * RB + rbo;
+            if (groupo < ngroups) {
+                const int o0 = 2 * p, o1 = 2 * p + 1 < NO ? 2 * p + 1 : 2 * p;
+                cx<T>* d0 = out + (o0 / ROWS) * ostride + (groupo * ROWS + o0 % ROWS) * (long)KC;
+                cx<T>* d1 = out + (o1 / ROWS) * ostride + (groupo * ROWS + o1 % ROWS) * (long)KC;
 #pragma unroll
                 for (int e = 0; e < EO; ++e) {
                     const int k = qo + PO * e;
@@ -398,17 +429,18 @@ k_rows_fused_pair(const cx<T>* __restrict__ in, long istride, cx<T>* __restrict_
 template <typename T, int L2, class PR>
 static void launch_fused_pair(mfic_ctx ctx, const void* in, void* out, long stride, int kc, long nrows, double scale,
                               const char* name) {
-    constexpr int NI = PR::NI, NO = PR::NO, GI = NI / 2;
+    constexpr int GI = pair_inputs<PR>();
     constexpr int RB = pair_rows_per_block<T, L2, GI>(), VI = pair_in_variant<T, L2>(), VO = pair_out_variant<T, L2, PR>();
-    MFIC_CHECK(3 * (kc - 1) == L2, MFIC_ERR_SIZE, "half-spectrum rows must hold N/2 + 1 values of a 3N/2 padded row");
+    MFIC_CHECK(3 * (kc - 1) == L2 && nrows % PR::ROWS == 0, MFIC_ERR_SIZE,
+               "half-spectrum rows must hold N/2 + 1 values of a 3N/2 padded row");
     const size_t lds = (size_t)RB * GI * pair_row_pitch<L2>() * sizeof(cx<T>);
     MFIC_CHECK(lds <= (size_t)ctx->max_lds, MFIC_ERR_SIZE, "fused row pass exceeds the LDS of a workgroup");
     const int prec = sizeof(T) == 8 ? MFIC_F64 : MFIC_F32;
     const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L2, 0, prec, VI));
     const cx<T>* two = static_cast<const cx<T>*>(twiddles(ctx, L2, 0, prec, VO));
-    dim3 grid((unsigned)xcd_grid((nrows + RB - 1) / RB));
+    dim3 grid((unsigned)xcd_grid((nrows / PR::ROWS + RB - 1) / RB));
     ProfScope prof(ctx, std::string(name) + "_n" + std::to_string(L2) + (sizeof(T) == 8 ? "_f64" : "_f32"),
-                   (double)nrows * (NI + NO) * kc * sizeof(cx<T>));
+                   (double)nrows * (PR::NF + PR::NOF) * kc * sizeof(cx<T>));
     hipLaunchKernelGGL((k_rows_fused_pair<T, L2, PR>), grid, dim3(pair_block_threads<T, L2, PR>()), lds, ctx->stream,
                        static_cast<const cx<T>*>(in), stride, static_cast<cx<T>*>(out), stride, nrows,
                        0.5 * scale * scale, tw, two);
@@ -418,7 +450,7 @@ static void launch_fused_pair(mfic_ctx ctx, const void* in, void* out, long stri
 template <typename T, int M, class PR>
 static void launch_fused(mfic_ctx ctx, const void* in, void* out, long stride, int kc, long nrows, double scale,
                          const char* name) {
-    constexpr int NI = PR::NI, NO = PR::NO, NG = NI / PR::IPG, SL = lane_slot<Plan<M>::P>();
+    constexpr int NI = PR::NF, NO = PR::NOF, NG = NI, SL = lane_slot<Plan<M>::P>();
     constexpr int RB = fused_rows_per_block<M, NG>(), RP = row_lds_pitch<M>();
     MFIC_CHECK(3 * (kc - 1) == 2 * M, MFIC_ERR_SIZE, "half-spectrum rows must hold N/2 + 1 values of a 3N/2 padded row");
     const size_t lds = (size_t)RB * NI * RP * sizeof(cx<T>);
@@ -442,12 +474,11 @@ static void launch_fused(mfic_ctx ctx, const void* in, void* out, long stride, i
 // group transforms one component row in LDS, then the row's particles are
 // written as interleaved FP64 [p][3], q + Psi for positions
 // ((ijk + shift)/N * lunit per axis, grid_fft.hh:242-252, not wrapped) or Psi
-// for velocities.
+// for velocities.  blockIdx.y takes the sets one after another.
+struct ParticleSets { ParticleRows s[8]; };
 template <typename T, int M>
 __global__ void __launch_bounds__((fused_rows_per_block<M, 3>() * 3 * lane_slot<Plan<M>::P>()))
-k_rows_c2r_particles(const cx<T>* __restrict__ f0, const cx<T>* __restrict__ f1, const cx<T>* __restrict__ f2,
-                     long nrows, T scale, const cx<T>* __restrict__ tw, double* __restrict__ dst, int is_pos,
-                     double lunit, double3 shift, size_t pbase) {
+k_rows_c2r_particles(ParticleSets sets, long nrows, T scale, const cx<T>* __restrict__ tw, double lunit) {
     constexpr int E = Plan<M>::E, P = Plan<M>::P, SL = lane_slot<P>(), N = 2 * M;
     constexpr int RP = row_lds_pitch<M>(), RB = fused_rows_per_block<M, 3>(), TPR = 3 * SL;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -462,7 +493,9 @@ k_rows_c2r_particles(const cx<T>* __restrict__ f0, const cx<T>* __restrict__ f1,
         // the untangle's partner M - k is loaded from global memory beside k
         // (same cache lines), so it runs in registers without an LDS round
         // trip (4.96 -> 4.13 ms for the four 512^3 launches)
-        const cx<T>* src = (g == 0 ? f0 : (g == 1 ? f1 : f2)) + (active ? row : 0) * (long)(M + 1);
+        const ParticleRows& ps = sets.s[blockIdx.y];
+        const cx<T>* __restrict__ src = static_cast<const cx<T>*>(g == 0 ? ps.f[0] : (g == 1 ? ps.f[1] : ps.f[2])) +
+                                        (active ? row : 0) * (long)(M + 1);
         cx<T> raw[E], rev[E], v[E];
 #pragma unroll
         for (int e = 0; e < E; ++e) {
@@ -487,14 +520,16 @@ k_rows_c2r_particles(const cx<T>* __restrict__ f0, const cx<T>* __restrict__ f1,
     __syncthreads();
     if (!active) return;
     const int i = (int)(row / N), j = (int)(row % N);
-    double* out = dst + 3 * (pbase + (size_t)row * N);
+    const bool is_pos = sets.s[blockIdx.y].is_pos != 0;
+    const double sh0 = sets.s[blockIdx.y].shift[0], sh1 = sets.s[blockIdx.y].shift[1], sh2 = sets.s[blockIdx.y].shift[2];
+    double* __restrict__ out = sets.s[blockIdx.y].dst + 3 * (size_t)row * N;
     for (int idx = tr; idx < 3 * N; idx += TPR) {
         const int p = idx / 3, c = idx - 3 * p;
         const cx<T> w = lds[(rb * 3 + c) * RP + (p >> 1)];
         double val = (double)((p & 1) ? w.y : w.x);
         if (is_pos) {
             const int ijk = c == 0 ? i : (c == 1 ? j : p);
-            const double sh = c == 0 ? shift.x : (c == 1 ? shift.y : shift.z);
+            const double sh = c == 0 ? sh0 : (c == 1 ? sh1 : sh2);
             val = (((double)ijk + sh) / (double)N) * lunit + val;
         }
         out[idx] = val;
@@ -502,8 +537,7 @@ k_rows_c2r_particles(const cx<T>* __restrict__ f0, const cx<T>* __restrict__ f1,
 }
 
 template <typename T, int M>
-static void launch_particles(mfic_ctx ctx, const void* const f[3], int is_pos, double lunit, const double shift[3],
-                             size_t pbase, double* dst) {
+static void launch_particles(mfic_ctx ctx, const ParticleSets& sets, int count, double lunit) {
     constexpr int SL = lane_slot<Plan<M>::P>(), RB = fused_rows_per_block<M, 3>(), RP = row_lds_pitch<M>();
     const long nrows = (long)(2 * M) * (2 * M);
     const size_t lds = (size_t)RB * 3 * RP * sizeof(cx<T>);
@@ -511,25 +545,22 @@ static void launch_particles(mfic_ctx ctx, const void* const f[3], int is_pos, d
     const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, M, 1, sizeof(T) == 8 ? MFIC_F64 : MFIC_F32));
     const double N = 2.0 * M;
     ProfScope prof(ctx, std::string("rows_c2r_particles_n") + std::to_string(2 * M) + (sizeof(T) == 8 ? "_f64" : "_f32"),
-                   (double)nrows * (3.0 * (M + 1) * sizeof(cx<T>) + 3.0 * 2 * M * 8.0));
-    dim3 grid((unsigned)((nrows + RB - 1) / RB));
-    hipLaunchKernelGGL((k_rows_c2r_particles<T, M>), grid, dim3(RB * 3 * SL), lds, ctx->stream,
-                       static_cast<const cx<T>*>(f[0]), static_cast<const cx<T>*>(f[1]),
-                       static_cast<const cx<T>*>(f[2]), nrows, (T)(1.0 / std::sqrt(N * N * N)), tw, dst, is_pos,
-                       lunit, make_double3(shift[0], shift[1], shift[2]), pbase);
+                   (double)nrows * (3.0 * (M + 1) * sizeof(cx<T>) + 3.0 * 2 * M * 8.0) * count);
+    const dim3 grid((unsigned)((nrows + RB - 1) / RB), count);
+    hipLaunchKernelGGL((k_rows_c2r_particles<T, M>), grid, dim3(RB * 3 * SL), lds, ctx->stream, sets, nrows,
+                       (T)(1.0 / std::sqrt(N * N * N)), tw, lunit);
     MFIC_LAUNCH_CHECK();
 }
 
 #define MFIC_PARTICLE_ROWS(X) X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384)
 
-void rows_c2r_particles(mfic_ctx ctx, int prec, const void* const f[3], int n, int is_pos, double lunit,
-                        const double shift[3], size_t pbase, double* dst) {
+template <typename T>
+void particle_rows(mfic_ctx ctx, const ParticleRows* sets, int count, int n, double lunit) {
+    MFIC_CHECK(count >= 1 && count <= 8, MFIC_ERR_ARG, "one to eight particle sets");
+    ParticleSets ps{};
+    for (int m = 0; m < count; ++m) ps.s[m] = sets[m];
     switch (n / 2) {
-#define X(M)                                                                                  \
-    case M:                                                                                   \
-        if (prec == MFIC_F64) launch_particles<double, M>(ctx, f, is_pos, lunit, shift, pbase, dst); \
-        else launch_particles<float, M>(ctx, f, is_pos, lunit, shift, pbase, dst);            \
-        break;
+#define X(M) case M: launch_particles<T, M>(ctx, ps, count, lunit); break;
         MFIC_PARTICLE_ROWS(X)
 #undef X
     default:
@@ -537,21 +568,23 @@ void rows_c2r_particles(mfic_ctx ctx, int prec, const void* const f[3], int n, i
     }
 }
 
+#ifndef MFIC_FUSED_SIZES
 #define MFIC_FUSED_SIZES(X) X(12) X(18) X(24) X(36) X(48) X(72) X(96) X(144) X(192) X(288) X(384) X(576) X(768)
+#endif
 
-template <typename T, class PR>
+template <typename T, class PR, bool HALF>
 static void fused_t(mfic_ctx ctx, size_t n, const void* in, void* out, const char* name) {
     const int N = (int)n, np = 3 * N / 2, kc = N / 2 + 1;
-    const long stride = (long)np * np * kc;
+    const long stride = (long)np * np * kc, rows = (long)np * np;
     const double norm = 1.0 / std::sqrt((double)np * (double)np * (double)np);
-    // form 0 (default): two rows per full-length transform; form 1: one
-    // half-length transform per row
-    const bool paired = plan_variant(ctx, np, MFIC_PASS_FUSED_ROWS, sizeof(T) == 8 ? MFIC_F64 : MFIC_F32) == 0;
+    // form 0 (default): two rows per full-length transform; form 1 (LPT
+    // sources only): one half-length transform per row
+    const bool paired = !HALF || plan_variant(ctx, np, MFIC_PASS_FUSED_ROWS, sizeof(T) == 8 ? MFIC_F64 : MFIC_F32) == 0;
     switch (np) {
-#define X(S)                                                                              \
-    case S:                                                                               \
-        if (paired) launch_fused_pair<T, S, PR>(ctx, in, out, stride, kc, (long)np * np, norm, name); \
-        else launch_fused<T, S / 2, PR>(ctx, in, out, stride, kc, (long)np * np, norm, name); \
+#define X(S)                                                                                    \
+    case S:                                                                                     \
+        if (paired) launch_fused_pair<T, S, PR>(ctx, in, out, stride, kc, rows, norm, name);    \
+        else if constexpr (HALF) launch_fused<T, S / 2, PR>(ctx, in, out, stride, kc, rows, norm, name); \
         break;
         MFIC_FUSED_SIZES(X)
 #undef X
@@ -560,24 +593,35 @@ static void fused_t(mfic_ctx ctx, size_t n, const void* in, void* out, const cha
     }
 }
 
-void fused_source_rows(mfic_ctx ctx, int prec, FusedKind kind, size_t n, const void* in, void* out) {
-    const bool f64 = prec == MFIC_F64;
+template <typename T> void fused_rows(mfic_ctx ctx, FusedKind kind, size_t n, const void* in, void* out) {
     switch (kind) {
-    case FusedKind::Src2:
-        f64 ? fused_t<double, ProdSrc2>(ctx, n, in, out, "fused_src2") : fused_t<float, ProdSrc2>(ctx, n, in, out, "fused_src2");
-        break;
-    case FusedKind::Src2Q:
-        f64 ? fused_t<double, ProdSrc2Q>(ctx, n, in, out, "fused_src2q") : fused_t<float, ProdSrc2Q>(ctx, n, in, out, "fused_src2q");
-        break;
-    case FusedKind::Src3:
-        f64 ? fused_t<double, ProdSrc3>(ctx, n, in, out, "fused_src3") : fused_t<float, ProdSrc3>(ctx, n, in, out, "fused_src3");
-        break;
+    case FusedKind::Src2: fused_t<T, ProdSrc2, true>(ctx, n, in, out, "fused_src2"); break;
+    case FusedKind::Src2Q: fused_t<T, ProdSrc2Q, true>(ctx, n, in, out, "fused_src2q"); break;
+    case FusedKind::Src3: fused_t<T, ProdSrc3, true>(ctx, n, in, out, "fused_src3"); break;
+    case FusedKind::Mul: fused_t<T, ProdMul, false>(ctx, n, in, out, "fused_mul"); break;
+    case FusedKind::Square: fused_t<T, ProdSquare, false>(ctx, n, in, out, "fused_square"); break;
+    case FusedKind::Adjoint2: fused_t<T, ProdAdjoint2, false>(ctx, n, in, out, "fused_adjoint2"); break;
     }
 }
 
-int fused_inputs(FusedKind kind) { return kind == FusedKind::Src3 ? ProdSrc3::NI : ProdSrc2::NI; }
-int fused_outputs(FusedKind kind) {
-    return kind == FusedKind::Src3 ? ProdSrc3::NO : kind == FusedKind::Src2Q ? ProdSrc2Q::NO : ProdSrc2::NO;
+#define MFIC_FUSED_T(MODE, T)                                                                                        \
+    MODE template void particle_rows<T>(mfic_ctx, const ParticleRows*, int, int, double);                            \
+    MODE template void fused_rows<T>(mfic_ctx, FusedKind, size_t, const void*, void*);
+
+#if MFIC_UNIT == 64
+MFIC_FUSED_T(, double)
+#else
+MFIC_FUSED_T(extern, double)
+
+void rows_c2r_particles(mfic_ctx ctx, int prec, const ParticleRows* sets, int count, int n, double lunit) {
+    if (prec == MFIC_F64) particle_rows<double>(ctx, sets, count, n, lunit);
+    else particle_rows<float>(ctx, sets, count, n, lunit);
 }
+
+void fused_source_rows(mfic_ctx ctx, int prec, FusedKind kind, size_t n, const void* in, void* out) {
+    if (prec == MFIC_F64) fused_rows<double>(ctx, kind, n, in, out);
+    else fused_rows<float>(ctx, kind, n, in, out);
+}
+#endif
 
 }  // namespace mfic

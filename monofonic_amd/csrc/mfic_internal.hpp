@@ -122,32 +122,41 @@ void require_device_memory(const void* p, const char* what);
 // the half-cell shift phases exp(i pi m / L), m < 2L (kind 2, FP64); the
 // inter-stage factors follow radix plan `variant` of the length
 const void* twiddles(mfic_ctx ctx, int L, int kind, int prec, int variant = 0);
-// the radix plan selected for a pass (mfic_fft_pass) of length L (0 unless
-// mfic_fft_set_plan chose another)
+// the radix plan selected for a pass (mfic_fft_pass) of length L: the default
+// of the pass unless mfic_fft_set_plan chose one
 int plan_variant(mfic_ctx ctx, int L, int pass, int prec);
 // number of radix plans compiled for length L
 int fft_plan_count(int L);
 // elements per thread and radices of plan `variant` of length L
 void fft_plan_info(int L, int variant, int* elems, int radices[4]);
 
-// FFT entry points on raw device buffers of layout [n0][n1][n2+2]
-template <typename T> void fft_r2c(mfic_ctx ctx, T* data, const size_t n[3], double scale);
-template <typename T> void fft_c2r(mfic_ctx ctx, T* data, const size_t n[3], double scale);
+// FFT entry points on raw device buffers of layout [n0][n1][n2+2]: `count`
+// grids of one size, each from src[m] to dst[m] (the same array or another)
+template <typename T>
+void fft_r2c(mfic_ctx ctx, const T* const* src, T* const* dst, int count, const size_t n[3], double scale);
+template <typename T>
+void fft_c2r(mfic_ctx ctx, const T* const* src, T* const* dst, int count, const size_t n[3], double scale);
+template <typename T> void fft_r2c(mfic_ctx ctx, T* data, const size_t n[3], double scale) {
+    fft_r2c<T>(ctx, &data, &data, 1, n, scale);
+}
+template <typename T> void fft_c2r(mfic_ctx ctx, T* data, const size_t n[3], double scale) {
+    fft_c2r<T>(ctx, &data, &data, 1, n, scale);
+}
 bool fft_length_supported(size_t n);
 
-// pass-level entry points used by fused pipelines
-template <typename T> void fft_c2r_cols(mfic_ctx ctx, T* data, const size_t n[3]);
-// fft_c2r_cols of a cubic-grid component plus, from the same axis-0 loads,
-// the component of the (1/2,1/2,1/2)-cell shifted sub-lattice into `shifted`;
-// with weights (wa, wb not null) the in-place output is shifted by wa / 2
-// and the second by wb / 2 cells per axis (0, 1 or 2 each)
+// the two strided c2r passes only (axis 0, axis 1), in place: the
+// contiguous-axis pass is left to a fused row kernel
+template <typename T> void fft_c2r_cols(mfic_ctx ctx, T* const* data, int count, const size_t n[3]);
+// fft_c2r_cols of cubic-grid components src[m] into data[m] plus, from the
+// same axis-0 loads, the components of the (1/2,1/2,1/2)-cell shifted
+// sub-lattice into shifted[m]; with weights (wa, wb not null) the first output
+// is shifted by wa / 2 and the second by wb / 2 cells per axis (0, 1 or 2
+// each).  src[m] may be data[m].
 template <typename T>
-void fft_c2r_cols_shift(mfic_ctx ctx, T* data, T* shifted, const size_t n[3], const int* wa = nullptr,
-                        const int* wb = nullptr);
-template <typename T> void fft_rows_r2c(mfic_ctx ctx, T* data, size_t nrows, int n2, double scale);
-template <typename T> void fft_rows_c2r(mfic_ctx ctx, T* data, size_t nrows, int n2, double scale);
-// complex pencils of length L: element (o, p, t) at data + o*os + p*ps + t,
-// t < tlen, o < nouter (offsets in complex elements)
+void fft_c2r_cols_shift(mfic_ctx ctx, const T* const* src, T* const* data, T* const* shifted, int count,
+                        const size_t n[3], const int* wa = nullptr, const int* wb = nullptr);
+// complex pencils of length L, in place: element (o, p, t) at data + o*os +
+// p*ps + t, t < tlen, o < nouter (offsets in complex elements)
 template <typename T>
 void fft_pencils(mfic_ctx ctx, void* data, int L, long ps, long os, int tlen, long nouter, bool fwd,
                  double scale, const char* tag = "");

@@ -1,7 +1,5 @@
 // Orszag 3/2 convolver core and the reorganised LPT source schedule.
 #pragma once
-#include <vector>
-
 #include "mfic_internal.hpp"
 
 namespace mfic {
@@ -10,6 +8,13 @@ struct OperandDesc {
     const void* f;  // k-space N-grid field (device)
     int kind;       // mfic_opkind
     int d[4];
+    bool same(const OperandDesc& o) const {
+        if (f != o.f || kind != o.kind) return false;
+        const int used = kind == MFIC_OPND_IDENT ? 0 : kind == MFIC_OPND_GRAD ? 1 : kind == MFIC_OPND_HESS ? 2 : 4;
+        for (int i = 0; i < used; ++i)
+            if (d[i] != o.d[i]) return false;
+        return true;
+    }
 };
 
 // Padded-grid operations for one N-grid size (OrszagConvolver, convolution.hh:412-651)
@@ -19,27 +24,15 @@ struct ConvCore {
     size_t N[3], Np[3];
     double len[3];
     ConvCore(mfic_ctx c, const size_t n[3], const double L[3], int prec);
-    size_t padded_reals() const;
     size_t grid_reals() const;
     size_t esize() const;
-    struct Term { const void* a; const void* b; double c; };
-    void pad_insert(const OperandDesc& o, void* fp) const;
-    void unpad(const void* fp, void* out, int op, double coef) const;
-    void c2r_padded(void* fp) const;
-    void r2c_padded(void* fp) const;
-    void mul(void* a, const void* b) const;
-    void prodsum(void* out, const std::vector<Term>& terms) const;
-    // buffer sizes (reals) of the pruned path: compact padded k buffer and a
-    // padded real field
+    // reals of a compact padded buffer ([Np][Np][N/2+1] complex)
     size_t kbuf_reals() const;
-    size_t real_reals() const;
-    void convolve2(const OperandDesc& a, const OperandDesc& b, void* out, int op, double coef, void* kbuf, void* r1,
-                   void* r2) const;
+    // kbuf: three compact buffers; fbuf: an N-grid
+    void convolve2(const OperandDesc& a, const OperandDesc& b, void* out, int op, double coef, void* kbuf) const;
     void convolve3(const OperandDesc& a, const OperandDesc& b, const OperandDesc& c, void* out, int op, double coef,
-                   void* kbuf, void* r1, void* r2, void* fbuf) const;
+                   void* kbuf, void* fbuf) const;
 };
-
-void add_inplace(mfic_ctx ctx, int prec, void* a, const void* b, size_t n);
 
 // phi2 (order >= 2), phi3 / A3 (order 3) from phi1, inverse Laplacian applied,
 // growth factors not applied

@@ -199,7 +199,9 @@ void plt_build(mfic_ctx ctx, int lat, int ng, PltTables& out) {
     MFIC_LAUNCH_CHECK();
     const size_t nn[3] = {(size_t)ng, (size_t)ng, (size_t)ng};
     const double norm = 1.0 / std::sqrt((double)ng * ng * ng);
-    for (int c = 0; c < 6; ++c) fft_r2c<double>(ctx, dD + c * nr, nn, norm);
+    double* comps[6];
+    for (int c = 0; c < 6; ++c) comps[c] = dD + c * nr;
+    fft_r2c<double>(ctx, comps, comps, 6, nn, norm);
     std::vector<double> hD(6 * nr);
     MFIC_HIP(hipMemcpyAsync(hD.data(), dD, 6 * nr * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     MFIC_HIP(hipStreamSynchronize(ctx->stream));

@@ -8,6 +8,8 @@
 // A complex grid is [n0][n1][n2] complex.  The c2c transform runs the
 // contiguous axis as row transforms in LDS and the two strided axes as the
 // pencil passes of the r2c/c2r transforms; both directions are unitary.
+//
+// This file is compiled once per precision (MFIC_UNIT 32 or 64).
 #include <cmath>
 #include <vector>
 
@@ -87,8 +89,11 @@ template <typename T> void fft_c2c(mfic_ctx ctx, void* data, const size_t n[3], 
                    "_c2c_ax1");
     fft_pencils<T>(ctx, data, (int)n[0], (long)(n[1] * n[2]), 0, (int)(n[1] * n[2]), 1, forward, scale, "_c2c_ax0");
 }
-template void fft_c2c<float>(mfic_ctx, void*, const size_t*, bool, double);
+#if MFIC_UNIT == 64
 template void fft_c2c<double>(mfic_ctx, void*, const size_t*, bool, double);
+#else
+template void fft_c2c<float>(mfic_ctx, void*, const size_t*, bool, double);
+#endif
 
 // ----------------------------------------------------------- PPT kernels --
 // Grid_FFT::get_k component of index i, in units of 2 pi / L (n/2 maps to
@@ -128,7 +133,7 @@ __global__ void k_ppt_maxdphi(const T* __restrict__ phi, int n, double* __restri
 // run on the elements of the transform passes beside them, and since i k_d
 // depends on one index only, the transforms of the other two axes cancel and
 // a gradient component is a forward and an inverse transform along its own
-// own axis.  HBM bound: 11 elements of psi read or written a cell (and 7 real
+// axis.  HBM bound: 11 elements of psi read or written a cell (and 7 real
 // values) where it took about 70.  The whole call at 192^3 FP64, order 2: 2.74
 // -> 0.69 ms, a third of it the two potentials' transforms; the passes run at
 // 3.2-4.5 TB/s, the ones with two transforms on a load the slowest.
@@ -172,7 +177,7 @@ k_ppt_rows_init(cx<T>* __restrict__ psi, const T* __restrict__ phi, const T* __r
 
 // exp(-i (hbar D+ / 2) k^2) for every index of one axis; the drift factor of
 // a mode is the product of its three
-__global__ void k_ppt_drift_table(cx<double>* __restrict__ tab, int n, double half_hbar_d, double kf) {
+static __global__ void k_ppt_drift_table(cx<double>* __restrict__ tab, int n, double half_hbar_d, double kf) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const double k = ppt_k(i, n) * kf;
@@ -393,6 +398,10 @@ void ppt_fields_t(mfic_ctx ctx, const PptInput& in, T* delta, T* vel[3], double*
     }
 }
 
+#if MFIC_UNIT == 64
+template void ppt_fields_t<double>(mfic_ctx, const PptInput&, double*, double*[3], double*);
+#else
+extern template void ppt_fields_t<double>(mfic_ctx, const PptInput&, double*, double*[3], double*);
 void ppt_fields(mfic_ctx ctx, int prec, const PptInput& in, void* delta, void* vel[3], double* hbar) {
     if (prec == MFIC_F64) {
         double* v[3] = {static_cast<double*>(vel[0]), static_cast<double*>(vel[1]), static_cast<double*>(vel[2])};
@@ -402,5 +411,6 @@ void ppt_fields(mfic_ctx ctx, int prec, const PptInput& in, void* delta, void* v
         ppt_fields_t<float>(ctx, in, static_cast<float*>(delta), v, hbar);
     }
 }
+#endif
 
 }  // namespace mfic
