@@ -57,8 +57,8 @@ class LPT2:
     def _padded(self, x):
         torch = _torch()
         n = self.n
-        buf = torch.zeros((n, n, n + 2), dtype=self._dtype(), device=x.device)
-        buf[:, :, :n] = x
+        buf = torch.empty((n, n, n + 2), dtype=self._dtype(), device=x.device)
+        buf[:, :, :n] = x  # the transforms do not read the pad columns
         return buf
 
     def _call(self, fn, tensors):

@@ -7,14 +7,16 @@
 #include <string>
 
 #include "cosmology.hpp"
+#include "fused.hpp"
 #include "kspace.hpp"
+#include "lpt.hpp"
 #include "mfic_internal.hpp"
 #include "orszag.hpp"
+#include "pruned.hpp"
 
 namespace mfic {
-void kspace_zero_nyquist(mfic_grid g);
-void kspace_grad_adjoint(mfic_grid out, mfic_grid gx, mfic_grid gy, mfic_grid gz, double unit);
-void kspace_hess_madd(mfic_grid out, mfic_grid r, int a, int b, double c);
+void kspace_grad_adjoint(mfic_grid lam, mfic_grid lmu, mfic_grid gx, mfic_grid gy, mfic_grid gz, double unit,
+                         double g2);
 }  // namespace mfic
 
 using mfic::Error;
@@ -40,11 +42,10 @@ struct mfic_lpt2_s {
     int prec = MFIC_F32;
     mfic::EhParams eh{};
     mfic_lpt_coef coef{};
-    GridPtr w, phi1, phi2, lam, lmu, r, t[3];
-    mfic_conv conv = nullptr;
+    GridPtr phi1, phi2, lam, lmu, t[3];
+    std::unique_ptr<mfic::ConvCore> core;  // sizes of the padded passes
     void* d_tk = nullptr;  // spline nodes of a tabulated transfer function
     ~mfic_lpt2_s() {
-        if (conv) (void)mfic_conv_destroy(conv);
         if (d_tk) (void)hipFree(d_tk);
     }
 };
@@ -60,14 +61,33 @@ void check_io(const mfic_lpt2_s* p, mfic_grid g, const char* what) {
     MFIC_CHECK(g->n[0] == p->n && g->n[1] == p->n && g->n[2] == p->n && g->prec == p->prec, MFIC_ERR_ARG,
                std::string("grid size / precision differs from the plan: ") + what);
 }
+// r2c of real grids into k-space grids of the plan
+template <typename T> void to_kspace(mfic_lpt2_s* p, mfic_grid* src, mfic_grid* dst, int count) {
+    const T* s[3];
+    T* d[3];
+    for (int m = 0; m < count; ++m) {
+        s[m] = static_cast<const T*>(src[m]->d);
+        d[m] = static_cast<T*>(dst[m]->d);
+        dst[m]->space = MFIC_KSPACE;
+    }
+    const size_t n3[3] = {p->n, p->n, p->n};
+    mfic::fft_r2c<T>(p->ctx, s, d, count, n3, 1.0 / std::sqrt((double)p->n * p->n * p->n));
+}
+// c2r in place
+template <typename T> void to_real(mfic_lpt2_s* p, mfic_grid* g, int count) {
+    T* d[3];
+    for (int m = 0; m < count; ++m) {
+        d[m] = static_cast<T*>(g[m]->d);
+        g[m]->space = MFIC_RSPACE;
+    }
+    const size_t n3[3] = {p->n, p->n, p->n};
+    mfic::fft_c2r<T>(p->ctx, d, d, count, n3, 1.0 / std::sqrt((double)p->n * p->n * p->n));
+}
 // phi1 = S P_N r2c(noise) (the forward map's first linear stage)
 void phi1_of(mfic_lpt2_s* p, mfic_grid noise) {
-    ck(mfic_grid_copy(p->w.g, noise));
-    ck(mfic_grid_set_space(p->w.g, MFIC_RSPACE));
-    ck(mfic_fft_forward(p->w.g));
-    mfic::kspace_zero_nyquist(p->w.g);
-    mfic::phi1_from_noise(p->phi1.g, p->w.g, p->eh, p->coef.volfac, 0, 0);
-    p->phi1.g->space = MFIC_KSPACE;
+    if (p->prec == MFIC_F64) to_kspace<double>(p, &noise, &p->phi1.g, 1);
+    else to_kspace<float>(p, &noise, &p->phi1.g, 1);
+    mfic::phi1_from_noise(p->phi1.g, p->phi1.g, p->eh, p->coef.volfac, 0, 0, nullptr, true);
 }
 }  // namespace
 
@@ -118,16 +138,14 @@ int mfic_lpt2_create(mfic_ctx ctx, size_t n, double L, int prec, const mfic_cosm
         }
         p->d_tk = mfic::tk_upload(*cosmo, &p->eh);
         ck(mfic_lpt_coefficients(cosmo, n, L, 2, &p->coef));
-        make(p.get(), p->w, MFIC_RSPACE);
         make(p.get(), p->phi1, MFIC_KSPACE);
         make(p.get(), p->phi2, MFIC_KSPACE);
         make(p.get(), p->lam, MFIC_KSPACE);
         make(p.get(), p->lmu, MFIC_KSPACE);
-        make(p.get(), p->r, MFIC_KSPACE);
-        for (auto& t : p->t) make(p.get(), t, MFIC_RSPACE);
+        for (auto& t : p->t) make(p.get(), t, MFIC_KSPACE);
         const size_t n3[3] = {n, n, n};
         const double L3[3] = {L, L, L};
-        ck(mfic_conv_create(ctx, n3, L3, prec, &p->conv));
+        p->core = std::make_unique<mfic::ConvCore>(ctx, n3, L3, prec);
         ++ctx->children;
         *out = p.release();
     });
@@ -151,11 +169,22 @@ int mfic_lpt2_forward(mfic_lpt2 p, mfic_grid noise, mfic_grid psi_x, mfic_grid p
         for (auto g : psi) check_io(p, g, "displacement");
         phi1_of(p, noise);
         mfic::lpt_sources(p->ctx, 2, p->phi1.g, p->phi2.g, nullptr, nullptr, nullptr, nullptr);
-        for (int d = 0; d < 3; ++d) {
-            ck(mfic_lpt_component(p->ctx, 2, d, &p->coef, nullptr, p->unit, p->phi1.g, p->phi2.g, nullptr, nullptr,
-                                  nullptr, nullptr, psi[d]));
-            ck(mfic_fft_backward(psi[d]));
-        }
+        // the three components in one pass over phi1 and phi2
+        const double cf[4] = {p->coef.g1, p->coef.g2, 0.0, 0.0};
+        const void* phi[3] = {p->phi1.g->d, p->phi2.g->d, nullptr};
+        const void* A3[3] = {nullptr, nullptr, nullptr};
+        // a buffer given for two components ends up with the later one
+        for (int d = 0; d < 2; ++d)
+            for (int e = d + 1; e < 3; ++e)
+                if (psi[d]->d == psi[e]->d) {
+                    psi[d]->space = MFIC_RSPACE;
+                    psi[d] = p->t[d].g;
+                    break;
+                }
+        void* outs[12] = {psi[0]->d, psi[1]->d, psi[2]->d};
+        mfic::assemble_all(p->ctx, p->prec, p->n, p->L, 2, cf, cf, p->unit, p->unit, mfic::PltDev{}, phi, A3, outs, 1);
+        if (p->prec == MFIC_F64) to_real<double>(p, psi, 3);
+        else to_real<float>(p, psi, 3);
     });
 }
 
@@ -168,38 +197,26 @@ int mfic_lpt2_adjoint(mfic_lpt2 p, mfic_grid noise, mfic_grid cot_x, mfic_grid c
         mfic_grid cot[3] = {cot_x, cot_y, cot_z};
         for (auto g : cot) check_io(p, g, "cotangent");
         phi1_of(p, noise);  // recomputed, not stored by the forward call
-        for (int d = 0; d < 3; ++d) {
-            ck(mfic_grid_copy(p->t[d].g, cot[d]));
-            ck(mfic_grid_set_space(p->t[d].g, MFIC_RSPACE));
-            ck(mfic_fft_forward(p->t[d].g));
-        }
-        // lam = unit sum_d (-i g_d) G_d (adjoint of the gradient, unit and DC := 0)
-        mfic::kspace_grad_adjoint(p->lam.g, p->t[0].g, p->t[1].g, p->t[2].g, p->unit);
-        // phi2 branch: lam_mu = P_N lap^-1 (g2 lam)
-        ck(mfic_grid_copy(p->lmu.g, p->lam.g));
-        ck(mfic_grid_scale(p->lmu.g, p->coef.g2));
-        ck(mfic_grid_inverse_laplacian(p->lmu.g));
-        mfic::kspace_zero_nyquist(p->lmu.g);
-        // phi1 branch
-        ck(mfic_grid_scale(p->lam.g, p->coef.g1));
-        // adjoint of the six Orszag products of the 2LPT source
-        mfic_operand L1{p->lmu.g, MFIC_OPND_IDENT, {0, 0, 0, 0}};
-        struct Term { int kind, d[4], a, b; double c; };
-        static const Term terms[6] = {
-            {MFIC_OPND_SUM_HESS, {1, 1, 2, 2}, 0, 0, 1.0}, {MFIC_OPND_SUM_HESS, {0, 0, 2, 2}, 1, 1, 1.0},
-            {MFIC_OPND_SUM_HESS, {0, 0, 1, 1}, 2, 2, 1.0}, {MFIC_OPND_HESS, {0, 1, 0, 0}, 0, 1, -2.0},
-            {MFIC_OPND_HESS, {0, 2, 0, 0}, 0, 2, -2.0},    {MFIC_OPND_HESS, {1, 2, 0, 0}, 1, 2, -2.0}};
-        for (const auto& t : terms) {
-            mfic_operand h{p->phi1.g, t.kind, {t.d[0], t.d[1], t.d[2], t.d[3]}};
-            ck(mfic_conv_convolve2(p->conv, &L1, &h, p->r.g, MFIC_OP_ASSIGN, 0.0));
-            mfic::kspace_hess_madd(p->lam.g, p->r.g, t.a, t.b, t.c);
-        }
-        // adjoint of phi1 = S P_N r2c(noise)
-        mfic::phi1_from_noise(p->w.g, p->lam.g, p->eh, p->coef.volfac, 0, 0);
-        p->w.g->space = MFIC_KSPACE;
-        mfic::kspace_zero_nyquist(p->w.g);
-        ck(mfic_fft_backward(p->w.g));
-        ck(mfic_grid_copy(grad, p->w.g));
+        mfic_grid t[3] = {p->t[0].g, p->t[1].g, p->t[2].g};
+        if (p->prec == MFIC_F64) to_kspace<double>(p, cot, t, 3);
+        else to_kspace<float>(p, cot, t, 3);
+        // lam = unit sum_d (-i g_d) G_d (adjoint of the gradient, unit and
+        // DC := 0) and lam_mu = P_N lap^-1 (g2 lam) of the phi2 branch
+        mfic::kspace_grad_adjoint(p->lam.g, p->lmu.g, t[0], t[1], t[2], p->unit, p->coef.g2);
+        // compact padded buffers: Hessians of phi1 [0, 6), lam_mu [6], the
+        // six products [7, 13); the x powers pass through [7, 10) on the way
+        // in and [0, 3) on the way out
+        const size_t kb = p->core->kbuf_reals() * p->core->esize();
+        char* ws = static_cast<char*>(mfic::ctx_scratch(p->ctx, "lpt2_adjoint", 13 * kb));
+        mfic::padded_hessians_to_kbuf(p->ctx, p->prec, p->phi1.g->d, p->n, p->L, ws + 7 * kb, ws);
+        const mfic::OperandDesc lmu{p->lmu.g->d, MFIC_OPND_IDENT, {0, 0, 0, 0}};
+        mfic::padded_operands_to_kbuf(p->ctx, p->prec, &lmu, 1, p->n, p->L, ws + 6 * kb);
+        mfic::fused_source_rows(p->ctx, p->prec, mfic::FusedKind::Adjoint2, p->n, ws, ws + 7 * kb);
+        // phi1 branch and the adjoint of phi1 = S P_N r2c(noise)
+        mfic::padded_hessian_adjoint(p->ctx, p->prec, p->n, p->L, ws + 7 * kb, ws, p->lam.g->d,
+                                     mfic::phi1_table(p->phi1.g, p->eh), p->coef.g1, p->coef.volfac, grad->d);
+        if (p->prec == MFIC_F64) to_real<double>(p, &grad, 1);
+        else to_real<float>(p, &grad, 1);
     });
 }
 

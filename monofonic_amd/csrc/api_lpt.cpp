@@ -696,10 +696,9 @@ int mfic_ppt_fields(mfic_run r, double velocity_unit, mfic_grid delta, mfic_grid
         const size_t nn[3] = {n, n, n};
         const double norm = 1.0 / std::sqrt((double)n * n * n);
         // growth-scaled real-space potentials (ic_generator.cc:644-658, 809, 847)
-        // and psi, in the workspace of the LPT sources (a run of order 2 or 3
-        // has one that is large enough)
+        // and psi, in a workspace of the context
         const size_t greal = n * n * (n + 2) * es, slot = (greal + 255) / 256 * 256;
-        char* ws = static_cast<char*>(ctx_scratch(r->ctx, "fused_in", 2 * slot + n * n * n * 2 * es));
+        char* ws = static_cast<char*>(ctx_scratch(r->ctx, "ppt_work", 2 * slot + n * n * n * 2 * es));
         void* ph1 = ws;
         void* ph2 = c.lpt_order >= 2 ? ws + slot : nullptr;
         // growth-scaled real-space potentials (ic_generator.cc:644-658, 809, 847)

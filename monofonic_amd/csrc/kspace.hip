@@ -115,11 +115,15 @@ __global__ void k_phi1_table(double* __restrict__ tab, int nmax, double kf, EhPa
 
 template <typename T>
 __global__ void k_phi1_tab(cx<T>* __restrict__ phi, const cx<T>* __restrict__ wn, const double* __restrict__ tab,
-                           KGeom G, size_t ncplx, double volfac, int fixing, int inversion) {
+                           KGeom G, size_t ncplx, double volfac, int fixing, int inversion, int zero_nyquist) {
     size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= ncplx) return;
     int i, j, k;
     G.ijk(idx, i, j, k);
+    if (zero_nyquist && (i == G.n0 / 2 || j == G.n1 / 2 || k == G.n2 / 2)) {
+        phi[idx] = cx<T>{0, 0};
+        return;
+    }
     const cx<T> w = wn[idx];
     double wr = w.x, wi = w.y;
     if (fixing) {
@@ -218,20 +222,23 @@ const double* phi1_table(mfic_grid phi, const EhParams& eh, double* table) {
 }
 
 void phi1_from_noise(mfic_grid phi, mfic_grid wn, const EhParams& eh, double volfac, int fixing, int inversion,
-                     double* table) {
+                     double* table, bool zero_nyquist) {
     MFIC_CHECK(eh.tk_n == 0 || eh.tk != nullptr, MFIC_ERR_STATE, "tabulated transfer function not on the device");
     const KGeom G = geom_of(phi);
     const size_t nc = (size_t)G.n0 * G.n1 * G.nc;
     const int bs = 256;
     ProfScope prof(phi->ctx, "phi1", 2.0 * phi->bytes());
+    MFIC_CHECK(!zero_nyquist || phi1_cubic(phi), MFIC_ERR_SIZE, "phi1 with empty Nyquist planes needs a cubic box");
     if (phi1_cubic(phi)) {
         const double* tab = phi1_table(phi, eh, table);
         if (phi->prec == MFIC_F64)
             hipLaunchKernelGGL(k_phi1_tab<double>, dim3(nblocks(nc, bs)), dim3(bs), 0, phi->ctx->stream,
-                               (cx<double>*)phi->d, (const cx<double>*)wn->d, tab, G, nc, volfac, fixing, inversion);
+                               (cx<double>*)phi->d, (const cx<double>*)wn->d, tab, G, nc, volfac, fixing, inversion,
+                               zero_nyquist ? 1 : 0);
         else
             hipLaunchKernelGGL(k_phi1_tab<float>, dim3(nblocks(nc, bs)), dim3(bs), 0, phi->ctx->stream,
-                               (cx<float>*)phi->d, (const cx<float>*)wn->d, tab, G, nc, volfac, fixing, inversion);
+                               (cx<float>*)phi->d, (const cx<float>*)wn->d, tab, G, nc, volfac, fixing, inversion,
+                               zero_nyquist ? 1 : 0);
         MFIC_LAUNCH_CHECK();
         return;
     }

@@ -408,6 +408,109 @@ k_hess_b(LdAx1<T, true> ld, StAx1<T, false> st, long ncols, T kf, const cx<T>* _
     }
 }
 
+// Adjoint of the Hessian passes, for sum_h D_h T(r_h) with D_h = -g_a g_b and
+// six real fields r_h given as r2c'd rows (slot order as the Hessians).  The
+// factors separate per axis, so pass B' sums the fields of an x power after
+// their axis-1 transforms, weighted by -g_j^q g_k^r, and pass A' the three
+// sums after theirs, weighted by g_i^p: three axis-0 transforms and one write
+// of the result for six of each.  Bound by memory: at 256^3 FP32 pass B' 291 us
+// (4.2 TB/s) for six fields, pass A' 160 us (2.8 TB/s; 16 columns to a tile,
+// whose factors and table reads are FP64), where one field took 63 + 45 us and
+// 58 us for its weighted sum.
+template <typename T, int L, int TK, int V>
+__global__ void __launch_bounds__((Plan<L, V>::P * TK))
+k_hess_bt(LdAx1<T, false> ld, StAx1<T, true> st, long ncols, T kf, const cx<T>* __restrict__ tw) {
+    using G = PadGeo<L, V>;
+    constexpr int E = Plan<L, V>::E;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
+    const int t = threadIdx.x % TK, q = threadIdx.x / TK;
+    const long col = xcd_tile(blockIdx.x, gridDim.x) * TK + t;
+    const bool active = col < ncols;
+    const long c = active ? col : 0;
+    const int first = HessOrder::first(blockIdx.y, 3), last = HessOrder::last(blockIdx.y, 3);
+    const T gk = grad_t<T>((int)(c % G::KC), G::N, kf);
+    cx<T> acc[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) acc[e] = cx<T>{0, 0};
+#pragma unroll 1
+    for (int i = first; i < last; ++i) {
+        const int pq = HessOrder::q(i), pr = HessOrder::r(i);
+        const T cm = pr == 0 ? T(-1) : (pr == 1 ? T(-1) * gk : T(-1) * (gk * gk));
+        const auto lc = ld.template column<L>(c, HessOrder::slot(i));
+        cx<T> v[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = ld.template load<L, V>(lc, q, e);
+        fft_pencil<T, L, true, V>(v, q, lds, LdsMap{t, TK}, tw);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const T g = G::template grad<T>(q, e, kf);  // band elements are not stored
+            const T m = cm * (pq > 0 ? g : T(1)) * (pq > 1 ? g : T(1));
+            acc[e] = cx<T>{acc[e].x + m * v[e].x, acc[e].y + m * v[e].y};
+        }
+    }
+    if (active) {
+        const auto sc = st.template column<L>(c, HessOrder::p(first));
+#pragma unroll
+        for (int e = 0; e < E; ++e) st.template store<L, V>(sc, q, e, acc[e]);
+    }
+}
+// out = F(|n|^2) / volfac * (g1 lam + scale * sum_p g_i^p (pass A' of slot p)),
+// Nyquist planes zeroed: F is the -A(k)/k^2 table of phi1
+template <typename T> struct AdjointOut {
+    cx<T>* out;
+    const cx<T>* lam;
+    const double* tab;
+    double g1, scale, volfac;
+};
+template <typename T, int L, int TK, int V>
+__global__ void __launch_bounds__((Plan<L, V>::P * TK))
+k_hess_at(LdPadCol<T> ld, AdjointOut<T> o, long ncols, T kf, const cx<T>* __restrict__ tw) {
+    using G = PadGeo<L, V>;
+    constexpr int E = Plan<L, V>::E;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
+    const int t = threadIdx.x % TK, q = threadIdx.x / TK;
+    const long col = (long)blockIdx.x * TK + t;
+    const bool active = col < ncols;
+    const long c = active ? col : 0;
+    cx<T> acc[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) acc[e] = cx<T>{0, 0};
+#pragma unroll 1
+    for (int p = 0; p < 3; ++p) {
+        const auto lc = ld.template column<L>(c, p);
+        cx<T> v[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = ld.template load<L, V>(lc, q, e);
+        fft_pencil<T, L, true, V>(v, q, lds, LdsMap{t, TK}, tw);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const T g = G::template grad<T>(q, e, kf);
+            const T m = (p > 0 ? g : T(1)) * (p > 1 ? g : T(1));
+            acc[e] = cx<T>{acc[e].x + m * v[e].x, acc[e].y + m * v[e].y};
+        }
+    }
+    if (!active) return;
+    const int j = (int)(c / G::KC), k = (int)(c % G::KC), sj = j - (j > G::NH) * G::N;
+    const bool nyq = j == G::NH || k == G::NH;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int i = G::src(q, e);
+        if (i < 0) continue;
+        const long at = (long)i * (G::N * G::KC) + c;
+        cx<T> r = {0, 0};
+        if (!nyq && i != G::NH) {
+            const int si = i - (i > G::NH) * G::N;
+            const double F = o.tab[si * si + sj * sj + k * k];
+            const cx<T> l = o.lam[at];
+            r = cx<T>{(T)((o.g1 * (double)l.x + o.scale * (double)acc[e].x) / o.volfac * F),
+                      (T)((o.g1 * (double)l.y + o.scale * (double)acc[e].y) / o.volfac * F)};
+        }
+        o.out[at] = r;
+    }
+}
+
 // Orszag truncation followed by re-padding along one axis of a compact
 // padded buffer that is real-space along that axis: forward transform, keep
 // the source modes (not the zero band, not the source Nyquist N/2), inverse
@@ -643,6 +746,57 @@ template <typename T> void hessians_to_kbuf(mfic_ctx ctx, const void* f, size_t 
 #undef X
 }
 
+template <typename T, int L, int V> static void launch_hess_bt(mfic_ctx ctx, const cx<T>* in, cx<T>* zb, T kf) {
+    constexpr int P = Plan<L, V>::P, N = 2 * L / 3, kc = N / 2 + 1;
+    const int tk = pick_tile<T, L, V>(ctx, MFIC_PASS_PAD_R2C_B, false);
+    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, 0, prec_of<T>(), V));
+    const long cols = (long)L * kc;
+    const dim3 grid((unsigned)xcd_grid((cols + tk - 1) / tk), 3);
+    ProfScope prof(ctx, pass_name<T, L>("fft_r2cBt"), (double)cols * (6 * L + 3 * N) * sizeof(cx<T>));
+#define CALL(K)                                                                                                \
+    hipLaunchKernelGGL((k_hess_bt<T, L, K, V>), grid, dim3(P * K), (size_t)L * K * sizeof(T), ctx->stream,     \
+                       LdAx1<T, false>{in}, StAx1<T, true>{zb}, cols, kf, tw);
+    MFIC_TILE_SWITCH(P, CALL)
+#undef CALL
+    MFIC_LAUNCH_CHECK();
+}
+template <typename T, int L, int V>
+static void launch_hess_at(mfic_ctx ctx, const cx<T>* zb, const AdjointOut<T>& o, T kf) {
+    constexpr int P = Plan<L, V>::P, N = 2 * L / 3, kc = N / 2 + 1;
+    const int tk = pick_tile<T, L, V>(ctx, MFIC_PASS_PAD_R2C_A, false);
+    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, 0, prec_of<T>(), V));
+    const long cols = (long)N * kc;
+    const dim3 grid((unsigned)((cols + tk - 1) / tk));
+    ProfScope prof(ctx, pass_name<T, L>("fft_r2cAt"), (double)cols * (3 * L + 2 * N) * sizeof(cx<T>));
+#define CALL(K)                                                                                                \
+    hipLaunchKernelGGL((k_hess_at<T, L, K, V>), grid, dim3(P * K), (size_t)L * K * sizeof(T), ctx->stream,     \
+                       LdPadCol<T>{zb}, o, cols, kf, tw);
+    MFIC_TILE_SWITCH(P, CALL)
+#undef CALL
+    MFIC_LAUNCH_CHECK();
+}
+
+template <typename T>
+void hessian_adjoint(mfic_ctx ctx, size_t n, double L, const void* prod, void* zbuf, const void* lam,
+                     const double* tab, double g1, double volfac, void* out) {
+    const int np = 3 * (int)n / 2;
+    const T kf = (T)(2.0 * 3.14159265358979323846 / L);
+    const double rfac = std::sqrt((double)np * np * np) / std::sqrt((double)n * n * n);
+    const double norm = 1.0 / std::sqrt((double)np * (double)np * (double)np);
+    const AdjointOut<T> o{static_cast<cx<T>*>(out), static_cast<const cx<T>*>(lam), tab, g1, norm / rfac, volfac};
+    cx<T>* zb = static_cast<cx<T>*>(zbuf);
+#define X(S)                                                                                                        \
+    case S:                                                                                                         \
+        if (plan_variant(ctx, S, MFIC_PASS_PAD_R2C_B, prec_of<T>()) == 1)                                           \
+            launch_hess_bt<T, S, alt_plan<S>()>(ctx, static_cast<const cx<T>*>(prod), zb, kf);                      \
+        else launch_hess_bt<T, S, 0>(ctx, static_cast<const cx<T>*>(prod), zb, kf);                                 \
+        if (plan_variant(ctx, S, MFIC_PASS_PAD_R2C_A, prec_of<T>()) == 1) launch_hess_at<T, S, alt_plan<S>()>(ctx, zb, o, kf); \
+        else launch_hess_at<T, S, 0>(ctx, zb, o, kf);                                                               \
+        break;
+    MFIC_PADDED_SWITCH(np)
+#undef X
+}
+
 template <typename T, int L, class LD, class ST, int V>
 static void launch_filter_v(mfic_ctx ctx, int pass, const LD& ld, const ST& st, long ncols, int members, bool xcd,
                             int zk, double scale, const char* name) {
@@ -692,6 +846,8 @@ template <typename T> void truncate_repad(mfic_ctx ctx, size_t n, void* kbuf, in
     MODE template void operands_to_kbuf<T>(mfic_ctx, const OperandDesc*, int, size_t, double, void*);                 \
     MODE template void r2c_from_kbuf<T>(mfic_ctx, size_t, double, void*, int, void* const*, int, double, bool);       \
     MODE template void hessians_to_kbuf<T>(mfic_ctx, const void*, size_t, double, void*, void*);                      \
+    MODE template void hessian_adjoint<T>(mfic_ctx, size_t, double, const void*, void*, const void*, const double*,   \
+                                          double, double, void*);                                                     \
     MODE template void truncate_repad<T>(mfic_ctx, size_t, void*, int);
 
 #if MFIC_UNIT == 64
@@ -702,6 +858,12 @@ MFIC_PRUNED_T(extern, double)
 void padded_hessians_to_kbuf(mfic_ctx ctx, int prec, const void* f, size_t n, double L, void* xbuf, void* out) {
     if (prec == MFIC_F64) hessians_to_kbuf<double>(ctx, f, n, L, xbuf, out);
     else hessians_to_kbuf<float>(ctx, f, n, L, xbuf, out);
+}
+
+void padded_hessian_adjoint(mfic_ctx ctx, int prec, size_t n, double L, const void* prod, void* zbuf, const void* lam,
+                            const double* tab, double g1, double volfac, void* out) {
+    if (prec == MFIC_F64) hessian_adjoint<double>(ctx, n, L, prod, zbuf, lam, tab, g1, volfac, out);
+    else hessian_adjoint<float>(ctx, n, L, prod, zbuf, lam, tab, g1, volfac, out);
 }
 
 void padded_truncate_repad(mfic_ctx ctx, int prec, size_t n, void* kbuf, int count) {

@@ -24,4 +24,12 @@ void padded_truncate_repad(mfic_ctx ctx, int prec, size_t n, void* kbuf, int cou
 void padded_r2c_from_kbuf(mfic_ctx ctx, int prec, size_t n, double L, void* kbuf, int count, void* const* out, int op,
                           double coef, bool invlap);
 
+// the adjoint of the Hessian passes with the last stage of the 2LPT adjoint:
+// six consecutive compact buffers of r2c'd rows (slot order as the Hessians)
+// -> out = F(|n|^2) / volfac (g1 lam + sum_h -g_a g_b T(r_h)) in k-space with
+// empty Nyquist planes, F the -A(k)/k^2 table of phi1_table; zbuf is scratch
+// for three compact buffers
+void padded_hessian_adjoint(mfic_ctx ctx, int prec, size_t n, double L, const void* prod, void* zbuf, const void* lam,
+                            const double* tab, double g1, double volfac, void* out);
+
 }  // namespace mfic
