@@ -211,15 +211,17 @@ k_rows_c2r(Fields<T> f, long nrows, long pitch, T scale, const cx<T>* __restrict
 #if MFIC_UNIT == 32
 // ------------------------------------------------------------ tables ------
 
-template <int L, int V = 0> static void fill_tw(std::vector<std::complex<long double>>& out) {
+// factor r (r = 1 .. R-1) of position k of a stage, k outermost or (rows) r
+// outermost
+template <int L, int V = 0> static void fill_tw(std::vector<std::complex<long double>>& out, bool rows) {
     const long double PI = 3.141592653589793238462643383279502884L;
     for (int s = 0; s < Plan<L, V>::S; ++s) {
         const int R = Plan<L, V>::r(s), NS = plan_ns<L, V>(s);
-        for (int k = 0; k < NS; ++k)
-            for (int r = 1; r < R; ++r) {
-                const long double a = -2.0L * PI * (long double)((long)r * k % ((long)NS * R)) / (long double)(NS * R);
-                out.emplace_back(cosl(a), sinl(a));
-            }
+        for (int i = 0; i < NS * (R - 1); ++i) {
+            const int k = rows ? i % NS : i / (R - 1), r = 1 + (rows ? i / NS : i % (R - 1));
+            const long double a = -2.0L * PI * (long double)((long)r * k % ((long)NS * R)) / (long double)(NS * R);
+            out.emplace_back(cosl(a), sinl(a));
+        }
     }
 }
 
@@ -288,13 +290,14 @@ static std::vector<std::complex<long double>> make_table(int L, int kind, int va
         }
         return tw;
     }
+    const bool rows = kind == 3;
     switch (L) {
 #define X(S)                                                     \
     case S:                                                      \
-        if (variant == 1) fill_tw<S, plan_or_default<S, 1>()>(tw);      \
-        else if (variant == 2) fill_tw<S, plan_or_default<S, 2>()>(tw); \
-        else if (variant == 3) fill_tw<S, plan_or_default<S, 3>()>(tw); \
-        else fill_tw<S>(tw);                                            \
+        if (variant == 1) fill_tw<S, plan_or_default<S, 1>()>(tw, rows);      \
+        else if (variant == 2) fill_tw<S, plan_or_default<S, 2>()>(tw, rows); \
+        else if (variant == 3) fill_tw<S, plan_or_default<S, 3>()>(tw, rows); \
+        else fill_tw<S>(tw, rows);                                            \
         break;
         MFIC_FOR_SIZES(X)
 #undef X
@@ -316,7 +319,7 @@ static std::vector<std::complex<long double>> make_table(int L, int kind, int va
 
 const void* twiddles(mfic_ctx ctx, int L, int kind, int prec, int variant) {
     std::lock_guard<std::mutex> lk(ctx->mu);
-    MFIC_CHECK(variant >= 0 && variant <= 3 && kind >= 0 && kind <= 2 && plan_exists(L, variant), MFIC_ERR_ARG,
+    MFIC_CHECK(variant >= 0 && variant <= 3 && kind >= 0 && kind <= 3 && plan_exists(L, variant), MFIC_ERR_ARG,
                "no such radix plan");
     auto key = std::make_tuple(L, kind + 4 * variant, prec);
     auto it = ctx->tables.find(key);

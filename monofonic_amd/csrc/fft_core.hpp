@@ -171,14 +171,16 @@ MFIC_PLAN(768, 24, 3, 12, 8, 8, 0)
 // alternatives of the padded-pass lengths: 16 threads per transform
 MFIC_PLAN_V(512, 1, 32, 3, 16, 8, 4, 0)
 MFIC_PLAN_V(768, 1, 48, 3, 16, 12, 4, 0)
-// row plan (V 2) for the output transforms of the 16-input fused pass: 32
-// threads per 384-point row
-MFIC_PLAN_V(384, 2, 12, 4, 12, 4, 4, 2)
-// row plans of the paired fused passes (two real rows per 768-point complex
-// transform): V 3 on 32 threads for the inputs, V 2 on 64 threads for the
-// outputs.  Radix orders with power-of-two spans before the last stage
-// (shift-and-mask twiddle indices) whose exchanges have conflict-free
-// swizzles.
+// row plans of the fused passes.  V 2, 12 values to a thread: 32 threads for
+// 384 points, 48 for 576, 64 for 768 (FP64 inputs, where 24 values fill the
+// registers, and outputs, of which there are few); V 3, 24 values to a thread
+// and half the threads (FP32 inputs).  Radix orders with power-of-two spans
+// where the length has them (shift-and-mask twiddle indices) and exchanges
+// that have conflict-free swizzles; no 24-point butterfly, whose temporaries
+// cost plan 0 of 384 (24 8 2) half its waves.
+MFIC_PLAN_V(384, 2, 12, 4, 4, 4, 4, 6)
+MFIC_PLAN_V(384, 3, 24, 3, 8, 8, 6, 0)
+MFIC_PLAN_V(576, 2, 12, 3, 4, 12, 12, 0)
 MFIC_PLAN_V(768, 2, 12, 4, 4, 4, 4, 12)
 MFIC_PLAN_V(768, 3, 24, 3, 8, 8, 12, 0)
 #undef MFIC_PLAN
@@ -192,14 +194,14 @@ template <int L> constexpr int alt_plan() { return plan_variants<L>() > 1 ? 1 : 
 template <int L> constexpr int row_alt_plan() { return L == 384 ? 2 : 0; }
 // whether plan V of length L is compiled (run-time form for table checks)
 __host__ __device__ constexpr bool plan_exists(int L, int V) {
-    return V == 0 || (V == 1 && (L == 512 || L == 768)) || (V == 2 && (L == 384 || L == 768)) || (V == 3 && L == 768);
+    return V == 0 || (V == 1 && (L == 512 || L == 768)) || (V == 2 && (L == 384 || L == 576 || L == 768)) ||
+           (V == 3 && (L == 384 || L == 768));
 }
 // plan V of L if compiled, else plan 0 (compile-time dispatch helper)
 template <int L, int V> constexpr int plan_or_default() { return plan_exists(L, V) ? V : 0; }
-// plans of the paired fused passes: input transforms (one group of lanes
-// per pair of input rows) and output transforms (one per pair of outputs)
-template <int L> constexpr int pair_in_plan() { return L == 768 ? 3 : 0; }
-template <int L> constexpr int pair_out_plan() { return L == 768 ? 2 : 0; }
+// plans of the paired fused passes: 24 values to a thread, or 12
+template <int L> constexpr int pair_narrow_plan() { return L == 768 || L == 384 ? 3 : 0; }
+template <int L> constexpr int pair_wide_plan() { return L == 768 || L == 576 || L == 384 ? 2 : 0; }
 
 template <int L, int V = 0> constexpr int plan_ns(int s) {  // span before stage s
     int ns = 1;
@@ -286,6 +288,15 @@ MFIC_SWZ_V(768, 1, 3, 1, 5, 0, 5, 4)
 MFIC_SWZ_V(768, 0, 2, 1, 4, 1, 6, 1)
 MFIC_SWZ_V(768, 1, 2, 1, 4, 1, 4, 4)
 MFIC_SWZ_V(768, 2, 2, 1, 6, 16, 6, 0)
+MFIC_SWZ_V(384, 0, 2, 1, 3, 1, 5, 1)
+MFIC_SWZ_V(384, 1, 2, 1, 4, 1, 4, 4)
+MFIC_SWZ_V(384, 2, 2, 1, 5, 0, 5, 8)
+MFIC_SWZ_V(576, 0, 2, 1, 3, 1, 5, 1)
+MFIC_SWZ_V(576, 1, 2, 1, 4, 0, 4, 4)
+MFIC_SWZ_V(384, 0, 3, 1, 3, 0, 4, 1)
+MFIC_SWZ_V(384, 1, 3, 1, 4, 0, 4, 2)
+MFIC_SWZ(576, 0, 1, 3, 1, 6, 1)
+MFIC_SWZ(576, 1, 1, 5, 0, 5, 4)
 #undef MFIC_SWZ
 #undef MFIC_SWZ_V
 __host__ __device__ constexpr bool pow2_or_0(int k) { return (k & (k - 1)) == 0; }
@@ -329,7 +340,10 @@ struct WaveSync {
 // SPLIT exchanges the real parts, then the imaginary parts, through an LDS
 // array of T: half the LDS of a complex exchange (more resident workgroups
 // for the wide pencil tiles) for twice the LDS instructions and barriers.
-template <typename T, int L, int S, bool FWD, class MAP, class SYNC = BlockSync, bool SPLIT = false, int V = 0>
+// Twiddle r of position k sits at k (R - 1) + r - 1, so that a thread's factors
+// come in wide loads, or (TWR) at (r - 1) NS + k, so that the lanes' factors of
+// one r sit side by side (a table in LDS: one conflict-free read for each r).
+template <typename T, int L, int S, bool FWD, class MAP, class SYNC = BlockSync, bool SPLIT = false, int V = 0, bool TWR = false>
 __device__ __forceinline__ void fft_stage(cx<T>* v, int q, cx<T>* lds, MAP m, const cx<T>* __restrict__ tw) {
     using PL = Plan<L, V>;
     constexpr int E = PL::E, P = PL::P, R = PL::r(S), B = E / R, NS = plan_ns<L, V>(S);
@@ -347,7 +361,7 @@ __device__ __forceinline__ void fft_stage(cx<T>* v, int q, cx<T>* lds, MAP m, co
         if (NS > 1) {
 #pragma unroll
             for (int r = 1; r < R; ++r) {
-                cx<T> w = tws[k * (R - 1) + (r - 1)];
+                cx<T> w = tws[TWR ? (r - 1) * NS + k : k * (R - 1) + (r - 1)];
                 a[r] = FWD ? cmul(a[r], w) : cmulc(a[r], w);
             }
         }
@@ -368,27 +382,30 @@ __device__ __forceinline__ void fft_stage(cx<T>* v, int q, cx<T>* lds, MAP m, co
     if constexpr (!LAST && SPLIT) {
         T* f = reinterpret_cast<T*>(lds);
 #pragma unroll
-        for (int b = 0; b < B; ++b) {
-            const int j = q + P * b;
-            const int base = (j / NS) * NS * R + j % NS;
+        for (int part = 0; part < 2; ++part) {
 #pragma unroll
-            for (int r = 0; r < R; ++r) f[m.at(base + r * NS)] = v[b + r * B].x;
+            for (int b = 0; b < B; ++b) {
+                const int j = q + P * b;
+                const int base = (j / NS) * NS * R + j % NS;
+                if constexpr (LINW) {
+                    const int fu = MAP::swz(base);
+#pragma unroll
+                    for (int r = 0; r < R; ++r) f[m.base + (fu ^ MAP::swz(r * NS))] = part ? v[b + r * B].y : v[b + r * B].x;
+                } else {
+#pragma unroll
+                    for (int r = 0; r < R; ++r) f[m.at(base + r * NS)] = part ? v[b + r * B].y : v[b + r * B].x;
+                }
+            }
+            SYNC::sync();
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                int at;
+                if constexpr (LINR) at = m.base + (MAP::swz(q) ^ MAP::swz(P * e));
+                else at = m.at(q + P * e);
+                (part ? v[e].y : v[e].x) = f[at];
+            }
+            SYNC::sync();
         }
-        SYNC::sync();
-#pragma unroll
-        for (int e = 0; e < E; ++e) v[e].x = f[m.at(q + P * e)];
-        SYNC::sync();
-#pragma unroll
-        for (int b = 0; b < B; ++b) {
-            const int j = q + P * b;
-            const int base = (j / NS) * NS * R + j % NS;
-#pragma unroll
-            for (int r = 0; r < R; ++r) f[m.at(base + r * NS)] = v[b + r * B].y;
-        }
-        SYNC::sync();
-#pragma unroll
-        for (int e = 0; e < E; ++e) v[e].y = f[m.at(q + P * e)];
-        SYNC::sync();
     } else if constexpr (!LAST && LINR) {  // q < P and P * e share no bits
         SYNC::sync();
         const int fq = MAP::swz(q);
@@ -500,18 +517,19 @@ __device__ __forceinline__ void fft_pencil2(cx<T>* v, cx<T>* w, int q, T* f, Lds
 }
 
 // full transform of a row held by one thread group, exchanges through the
-// per-stage swizzled LDS slots starting at `base`
-template <typename T, int L, bool FWD, class SYNC = BlockSync, int V = 0>
+// per-stage swizzled LDS slots starting at `base` (with SPLIT in units of T,
+// real and imaginary parts in turn)
+template <typename T, int L, bool FWD, class SYNC = BlockSync, int V = 0, bool SPLIT = false, bool TWR = false>
 __device__ __forceinline__ void fft_regs_row(cx<T>* v, int q, cx<T>* lds, int base, const cx<T>* __restrict__ tw) {
     constexpr int S = Plan<L, V>::S;
     using M0 = LdsSwzMap<L, 0, V>;
     using M1 = LdsSwzMap<L, 1 % S, V>;
     using M2 = LdsSwzMap<L, 2 % S, V>;
     using M3 = LdsSwzMap<L, 3 % S, V>;
-    fft_stage<T, L, 0, FWD, M0, SYNC, false, V>(v, q, lds, M0{base}, tw);
-    if constexpr (S > 1) fft_stage<T, L, 1 % S, FWD, M1, SYNC, false, V>(v, q, lds, M1{base}, tw);
-    if constexpr (S > 2) fft_stage<T, L, 2 % S, FWD, M2, SYNC, false, V>(v, q, lds, M2{base}, tw);
-    if constexpr (S > 3) fft_stage<T, L, 3 % S, FWD, M3, SYNC, false, V>(v, q, lds, M3{base}, tw);
+    fft_stage<T, L, 0, FWD, M0, SYNC, SPLIT, V, TWR>(v, q, lds, M0{base}, tw);
+    if constexpr (S > 1) fft_stage<T, L, 1 % S, FWD, M1, SYNC, SPLIT, V, TWR>(v, q, lds, M1{base}, tw);
+    if constexpr (S > 2) fft_stage<T, L, 2 % S, FWD, M2, SYNC, SPLIT, V, TWR>(v, q, lds, M2{base}, tw);
+    if constexpr (S > 3) fft_stage<T, L, 3 % S, FWD, M3, SYNC, SPLIT, V, TWR>(v, q, lds, M3{base}, tw);
 }
 
 }  // namespace mfic

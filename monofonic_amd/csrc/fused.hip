@@ -82,17 +82,17 @@ struct ProdSrc3 {
 };
 // convolver products: two operands, or one with itself
 struct ProdMul {
-    static constexpr int NF = 2, NOF = 1, ROWS = 2, WAVES = 3;
+    static constexpr int NF = 2, NOF = 1, ROWS = 2;
     __device__ static __forceinline__ void eval(const double* h, double* o) { o[0] = h[0] * h[1]; }
 };
 struct ProdSquare {
-    static constexpr int NF = 1, NOF = 1, ROWS = 2, WAVES = 3;
+    static constexpr int NF = 1, NOF = 1, ROWS = 2;
     __device__ static __forceinline__ void eval(const double* h, double* o) { o[0] = h[0] * h[0]; }
 };
 // adjoint of the 2LPT source: phi1 Hessians a[0..5] and lambda [6] -> lambda
 // times the derivative of the source with respect to each Hessian
 struct ProdAdjoint2 {
-    static constexpr int NF = 7, NOF = 6, ROWS = 2, WAVES = 3;
+    static constexpr int NF = 7, NOF = 6, ROWS = 2;
     __device__ static __forceinline__ void eval(const double* a, double* o) {
         const double l = a[6];
         o[0] = l * (a[1] + a[2]);
@@ -258,51 +258,62 @@ k_rows_fused(const cx<T>* __restrict__ in, long istride, cx<T>* __restrict__ out
 // forward transform as O_2p[k] = W[k] + conj(W[L2-k]),
 // O_2p+1[k] = -i (W[k] - conj(W[L2-k])) (the 1/2 and both normalisations
 // are one FP64 factor on the products).
-// input transforms on the 32-lane plan; FP64 on the 64-lane output plan
-// (twice the wavefronts per row: the FP64 passes hold one or two workgroups
-// per CU, so their latency wants the waves)
-template <typename T, int L2> constexpr int pair_in_variant() {
-    return sizeof(T) == 8 && pair_out_plan<L2>() != 0 ? pair_out_plan<L2>() : pair_in_plan<L2>();
+//
+// Bound by vector issue and by latency: 65% of the issue slots at 3 waves a
+// SIMD, which is what whole complex rows in LDS left room for.  So an exchange
+// takes real and imaginary parts in turn and the product stage half the
+// points at a time, which halves the LDS (4 waves and more), the factors
+// between stages are read from LDS (from memory, the lanes' spread-out reads
+// of them kept the vector cache busier than the data), and the plans avoid
+// the 24-point butterfly.  6-, 16- and 7-input passes:
+//   768 FP32 4.37 -> 3.97 ms, 8.79 -> 7.2 ms; 384 FP32 0.62 -> 0.46, 1.11 ->
+//   0.82, 0.73 -> 0.53 ms; 288 FP64 0.48 -> 0.45, 0.85 -> 0.76 ms; 384 FP64
+//   1.45 -> 0.95, 2.79 -> 1.63 ms; 576 FP64 5.36 -> 4.07, 9.30 -> 6.73 ms
+// without the transforms the same loads and stores take 5.1 ms (768, 16
+// inputs), 0.76 (384) and 0.56 (288 FP64).
+template <typename T, int L2> constexpr int pair_variant() {
+    // 24 values to a thread in FP32 (576 points, which have no plan of that
+    // kind with power-of-two spans: 12), 12 in FP64
+    return sizeof(T) == 8 || L2 == 576 ? pair_wide_plan<L2>() : pair_narrow_plan<L2>();
+}
+// waves per SIMD to fit the registers to: 4 hold 12 FP64 or 24 FP32 values
+// without spilling (288 points FP64, 16 inputs: 0.76 ms, 0.88 with the
+// compiler's own choice of 3), except for four-stage FP64 plans with their
+// precomputed exchange addresses (384 points, 2 inputs: 0.27 ms with 3, 0.31
+// with 4)
+template <typename T, int L2> constexpr int pair_waves() {
+    return sizeof(T) == 8 && Plan<L2, pair_variant<T, L2>()>::S > 3 ? 3 : 4;
 }
 template <typename T, int L2, int GI> constexpr int pair_rows_per_block() {
-    constexpr int tpr = GI * lane_slot<Plan<L2, pair_in_variant<T, L2>()>::P>();
+    constexpr int tpr = GI * lane_slot<Plan<L2, pair_variant<T, L2>()>::P>();
     return tpr >= 256 ? 1 : (256 / tpr > 8 ? 8 : 256 / tpr);
 }
 template <class PR> constexpr int pair_inputs() { return PR::NF * PR::ROWS / 2; }
 template <class PR> constexpr int pair_outputs() { return (PR::NOF * PR::ROWS + 1) / 2; }
 template <typename T, int L2, class PR> constexpr int pair_block_threads() {
     constexpr int GI = pair_inputs<PR>();
-    return pair_rows_per_block<T, L2, GI>() * GI * lane_slot<Plan<L2, pair_in_variant<T, L2>()>::P>();
+    return pair_rows_per_block<T, L2, GI>() * GI * lane_slot<Plan<L2, pair_variant<T, L2>()>::P>();
 }
-// output transforms on 64 lanes (plan pair_out_plan) where every output
-// pair of the block gets a wavefront, else on the input transforms' lanes
-template <typename T, int L2, class PR> constexpr int pair_out_variant() {
-    constexpr int GO = pair_outputs<PR>(), RB = pair_rows_per_block<T, L2, pair_inputs<PR>()>();
-    constexpr int VO = pair_out_plan<L2>();
-    return VO != 0 && RB * GO * lane_slot<Plan<L2, VO>::P>() <= pair_block_threads<T, L2, PR>() ? VO
-                                                                                               : pair_in_variant<T, L2>();
-}
-
-// LDS slots per pair row: the first pitch of at least L2 that is 32 modulo
-// 64, so the two rows a wavefront covers (two 32-lane groups) fall on
-// opposite halves of the 64 bank slots
-template <int L2> constexpr int pair_row_pitch() { return L2 + ((32 - L2 % 64) % 64 + 64) % 64; }
+// LDS of a pair row, in T: an exchange takes real and imaginary parts in turn
+// and the product stage half the points at a time, so a row needs L2 values
+// of T, not L2 complex ones.  The pitch puts the transforms that share a
+// 32-lane group a lane slot apart modulo the 32 banks.
+template <int L2, int SL> constexpr int pair_row_pitch() { return L2 + (((SL < 2 ? 2 : SL) - L2) % 32 + 32) % 32; }
 
 template <typename T, int L2, class PR>
 __global__ void __launch_bounds__((pair_block_threads<T, L2, PR>()))
-__attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? PR::WAVES : 1, 8)))
+__attribute__((amdgpu_waves_per_eu(pair_waves<T, L2>(), 8)))
 k_rows_fused_pair(const cx<T>* __restrict__ in, long istride, cx<T>* __restrict__ out, long ostride, long nrows,
-                  double scale2, const cx<T>* __restrict__ tw, const cx<T>* __restrict__ two) {
+                  double scale2, const cx<T>* __restrict__ tw) {
     constexpr int NF = PR::NF, NOF = PR::NOF, ROWS = PR::ROWS, NI = NF * ROWS, NO = NOF * ROWS;
     constexpr int GI = pair_inputs<PR>(), GO = pair_outputs<PR>();
-    constexpr int VI = pair_in_variant<T, L2>(), VO = pair_out_variant<T, L2, PR>();
-    constexpr int E = Plan<L2, VI>::E, P = Plan<L2, VI>::P, SL = lane_slot<P>();
-    constexpr int EO = Plan<L2, VO>::E, PO = Plan<L2, VO>::P, SLO = lane_slot<PO>();
-    constexpr int RB = pair_rows_per_block<T, L2, GI>(), TPR = GI * SL, RP = pair_row_pitch<L2>();
+    constexpr int V = pair_variant<T, L2>(), E = Plan<L2, V>::E, P = Plan<L2, V>::P, SL = lane_slot<P>();
+    constexpr int RB = pair_rows_per_block<T, L2, GI>(), TPR = GI * SL, RP = pair_row_pitch<L2, SL>();
     constexpr int KC = L2 / 3 + 1;  // N/2 + 1 values per compact row, N = 2 L2 / 3
-    constexpr int NPOS = (L2 + TPR - 1) / TPR;
+    constexpr int H = L2 / 2, HP = RP / 2, NPOS = (H + TPR - 1) / TPR;
+    static_assert(E % 2 == 0 && L2 % 2 == 0 && RP % 2 == 0, "rows are handled in halves");
     static_assert(NI % 2 == 0, "inputs come in pairs");
-    static_assert(P <= 64 && PO <= 64 && 64 % SL == 0 && 64 % SLO == 0, "a transform must fit in one wavefront");
+    static_assert(P <= 64 && 64 % SL == 0, "a transform must fit in one wavefront");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
     const int tr = threadIdx.x % TPR, rb = threadIdx.x / TPR;
@@ -312,14 +323,22 @@ k_rows_fused_pair(const cx<T>* __restrict__ in, long istride, cx<T>* __restrict_
     const long tile = xcd_tile(blockIdx.x, gridDim.x);
     const long group = tile * RB + rb, ngroups = nrows / ROWS;
 
+    // the inter-stage factors go to LDS once for the block: read from memory
+    // by every lane they cost more cycles in the vector cache than the data
+    constexpr int NTW = plan_tw_size<L2, V>(), NT = pair_block_threads<T, L2, PR>();
+    cx<T>* ltw = lds + RB * GI * HP;
+#pragma unroll
+    for (int i = 0; i < NTW; i += NT)
+        if (i + (int)threadIdx.x < NTW) ltw[i + threadIdx.x] = tw[i + threadIdx.x];
+
     // 1. inverse transform of input pair g: all compact-row loads first, the
     // zero band (N/2 < k < L2 - N/2) never loaded
+    cx<T> v[E], a[E], b[E];
     if (q < P) {
         const long r0 = (group < ngroups ? group : 0) * (long)(ROWS * KC);
         const int i0 = 2 * g, i1 = 2 * g + 1;
         const cx<T>* s0 = in + (i0 / ROWS) * istride + r0 + (i0 % ROWS) * KC;
         const cx<T>* s1 = in + (i1 / ROWS) * istride + r0 + (i1 % ROWS) * KC;
-        cx<T> a[E], b[E];
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const int k = q + P * e;
@@ -340,7 +359,9 @@ k_rows_fused_pair(const cx<T>* __restrict__ in, long istride, cx<T>* __restrict_
                 }
             }
         }
-        cx<T> v[E];
+    }
+    __syncthreads();
+    if (q < P) {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const int k = q + P * e;
@@ -351,76 +372,92 @@ k_rows_fused_pair(const cx<T>* __restrict__ in, long istride, cx<T>* __restrict_
                 v[e] = cx<T>{a[e].x - b[e].y, a[e].y + b[e].x};  // A + i B
             }
         }
-        const int base = (rb * GI + g) * RP;
-        fft_regs_row<T, L2, false, WaveSync, VI>(v, q, lds, base, tw);
-#pragma unroll
-        for (int e = 0; e < E; ++e) lds[base + q + P * e] = v[e];
+        fft_regs_row<T, L2, false, WaveSync, V, true, true>(v, q, lds, (rb * GI + g) * RP, ltw);
     }
-    __syncthreads();
 
     // 2. products at every real point n from the NI/2 pair rows, in FP64,
-    // times the normalisation; outputs paired over the first pair rows (a
-    // point is read and written by one thread only)
+    // times the normalisation, half the points at a time; outputs paired over
+    // the first pair rows (a point is read and written by one thread only)
+    // and taken by their transforms' threads
+    const int rbo = (threadIdx.x / SL) / GO, po = (threadIdx.x / SL) % GO;
+    // the position again, as a value of its own: or the compiler holds the
+    // inverse transforms' factors and addresses in registers for the forward
+    // ones and spills (768 points, 6 inputs: 5.0 against 4.0 ms)
+    int qo = q;
+    asm("" : "+v"(qo));
+    const bool olane = rbo < RB && qo < P;
+    const int obase = (rbo * GI + po) * HP;
+    cx<T> w[E];
 #pragma unroll
-    for (int u = 0; u < NPOS; ++u) {
-        const int n = tr + u * TPR;
-        if (n < L2) {
-            double h[NI], o[NO];
+    for (int half = 0; half < 2; ++half) {
+        if (q < P) {
+            const int base = (rb * GI + g) * HP;
 #pragma unroll
-            for (int p = 0; p < GI; ++p) {
-                const cx<T> z = lds[(rb * GI + p) * RP + n];
-                h[2 * p] = (double)z.x;
-                h[2 * p + 1] = (double)z.y;
-            }
+            for (int e = 0; e < E / 2; ++e) lds[base + q + P * e] = v[e + half * (E / 2)];
+        }
+        __syncthreads();
+        // the second half starts half a row of threads on, where the first
+        // half's last round may have left threads without a point
+        const int t0 = half ? (tr + TPR / 2) % TPR : tr;
 #pragma unroll
-            for (int r = 0; r < ROWS; ++r) {
-                double hr[NF], orow[NOF];
+        for (int u = 0; u < NPOS; ++u) {
+            const int n = t0 + u * TPR;
+            if (n < H) {
+                double h[NI], o[NO];
 #pragma unroll
-                for (int f = 0; f < NF; ++f) hr[f] = h[f * ROWS + r];
-                PR::eval(hr, orow);
+                for (int p = 0; p < GI; ++p) {
+                    const cx<T> z = lds[(rb * GI + p) * HP + n];
+                    h[2 * p] = (double)z.x;
+                    h[2 * p + 1] = (double)z.y;
+                }
 #pragma unroll
-                for (int f = 0; f < NOF; ++f) o[f * ROWS + r] = orow[f];
-            }
+                for (int r = 0; r < ROWS; ++r) {
+                    double hr[NF], orow[NOF];
 #pragma unroll
-            for (int p = 0; p < GO; ++p) {
-                const T lo = (T)(o[2 * p] * scale2);
-                const T hi = 2 * p + 1 < NO ? (T)(o[2 * p + 1] * scale2) : (T)0;
-                lds[(rb * GI + p) * RP + n] = cx<T>{lo, hi};
+                    for (int f = 0; f < NF; ++f) hr[f] = h[f * ROWS + r];
+                    PR::eval(hr, orow);
+#pragma unroll
+                    for (int f = 0; f < NOF; ++f) o[f * ROWS + r] = orow[f];
+                }
+#pragma unroll
+                for (int p = 0; p < GO; ++p) {
+                    const T lo = (T)(o[2 * p] * scale2);
+                    const T hi = 2 * p + 1 < NO ? (T)(o[2 * p + 1] * scale2) : (T)0;
+                    lds[(rb * GI + p) * HP + n] = cx<T>{lo, hi};
+                }
             }
         }
+        __syncthreads();
+        if (olane) {
+#pragma unroll
+            for (int e = 0; e < E / 2; ++e) w[e + half * (E / 2)] = lds[obase + qo + P * e];
+        }
+        if (half == 0) __syncthreads();
     }
-    __syncthreads();
 
-    // 3. forward transform of output pair p, separated into the two outputs'
+    // 3. forward transform of output pair po, separated into the two outputs'
     // first KC modes
-    {
-        const int t = threadIdx.x / SLO, qo = threadIdx.x % SLO;
-        const int rbo = t / GO, p = t % GO;
-        if (t < RB * GO && qo < PO) {
-            const int base = (rbo * GI + p) * RP;
-            cx<T> v[EO];
+    if (olane) {
+        WaveSync::sync();
+        fft_regs_row<T, L2, true, WaveSync, V, true, true>(w, qo, lds, 2 * obase, ltw);
+        // partners W[L2 - k] of the kept modes sit at L2 - KC + 1 .. L2 - 1,
+        // in the upper half of the row
 #pragma unroll
-            for (int e = 0; e < EO; ++e) v[e] = lds[base + qo + PO * e];
-            WaveSync::sync();
-            fft_regs_row<T, L2, true, WaveSync, VO>(v, qo, lds, base, two);
-            // partners W[L2 - k] of the kept modes sit at L2 - KC + 1 .. L2 - 1
+        for (int e = E / 2; e < E; ++e)
+            if (P * e + P > L2 - KC + 1) lds[obase + qo + P * e - H] = w[e];
+        WaveSync::sync();
+        const long groupo = tile * RB + rbo;
+        if (groupo < ngroups) {
+            const int o0 = 2 * po, o1 = 2 * po + 1 < NO ? 2 * po + 1 : 2 * po;
+            cx<T>* d0 = out + (o0 / ROWS) * ostride + (groupo * ROWS + o0 % ROWS) * (long)KC;
+            cx<T>* d1 = out + (o1 / ROWS) * ostride + (groupo * ROWS + o1 % ROWS) * (long)KC;
 #pragma unroll
-            for (int e = 0; e < EO; ++e)
-                if (PO * e + PO > L2 - KC + 1) lds[base + qo + PO * e] = v[e];
-            WaveSync::sync();
-            const long groupo = tile * RB + rbo;
-            if (groupo < ngroups) {
-                const int o0 = 2 * p, o1 = 2 * p + 1 < NO ? 2 * p + 1 : 2 * p;
-                cx<T>* d0 = out + (o0 / ROWS) * ostride + (groupo * ROWS + o0 % ROWS) * (long)KC;
-                cx<T>* d1 = out + (o1 / ROWS) * ostride + (groupo * ROWS + o1 % ROWS) * (long)KC;
-#pragma unroll
-                for (int e = 0; e < EO; ++e) {
-                    const int k = qo + PO * e;
-                    if (PO * e >= KC || k >= KC) continue;
-                    const cx<T> w = v[e], wm = k == 0 ? v[e] : lds[base + L2 - k];
-                    d0[k] = cx<T>{w.x + wm.x, w.y - wm.y};
-                    if (2 * p + 1 < NO) d1[k] = cx<T>{w.y + wm.y, wm.x - w.x};
-                }
+            for (int e = 0; e < E; ++e) {
+                const int k = qo + P * e;
+                if (P * e >= KC || k >= KC) continue;
+                const cx<T> x = w[e], xm = k == 0 ? w[e] : lds[obase + H - k];
+                d0[k] = cx<T>{x.x + xm.x, x.y - xm.y};
+                if (2 * po + 1 < NO) d1[k] = cx<T>{x.y + xm.y, xm.x - x.x};
             }
         }
     }
@@ -430,20 +467,20 @@ template <typename T, int L2, class PR>
 static void launch_fused_pair(mfic_ctx ctx, const void* in, void* out, long stride, int kc, long nrows, double scale,
                               const char* name) {
     constexpr int GI = pair_inputs<PR>();
-    constexpr int RB = pair_rows_per_block<T, L2, GI>(), VI = pair_in_variant<T, L2>(), VO = pair_out_variant<T, L2, PR>();
+    constexpr int RB = pair_rows_per_block<T, L2, GI>(), V = pair_variant<T, L2>();
     MFIC_CHECK(3 * (kc - 1) == L2 && nrows % PR::ROWS == 0, MFIC_ERR_SIZE,
                "half-spectrum rows must hold N/2 + 1 values of a 3N/2 padded row");
-    const size_t lds = (size_t)RB * GI * pair_row_pitch<L2>() * sizeof(cx<T>);
+    constexpr int RP = pair_row_pitch<L2, lane_slot<Plan<L2, V>::P>()>();
+    const size_t lds = (size_t)RB * GI * RP * sizeof(T) + plan_tw_size<L2, V>() * sizeof(cx<T>);
     MFIC_CHECK(lds <= (size_t)ctx->max_lds, MFIC_ERR_SIZE, "fused row pass exceeds the LDS of a workgroup");
     const int prec = sizeof(T) == 8 ? MFIC_F64 : MFIC_F32;
-    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L2, 0, prec, VI));
-    const cx<T>* two = static_cast<const cx<T>*>(twiddles(ctx, L2, 0, prec, VO));
+    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L2, 3, prec, V));
     dim3 grid((unsigned)xcd_grid((nrows / PR::ROWS + RB - 1) / RB));
     ProfScope prof(ctx, std::string(name) + "_n" + std::to_string(L2) + (sizeof(T) == 8 ? "_f64" : "_f32"),
                    (double)nrows * (PR::NF + PR::NOF) * kc * sizeof(cx<T>));
     hipLaunchKernelGGL((k_rows_fused_pair<T, L2, PR>), grid, dim3(pair_block_threads<T, L2, PR>()), lds, ctx->stream,
                        static_cast<const cx<T>*>(in), stride, static_cast<cx<T>*>(out), stride, nrows,
-                       0.5 * scale * scale, tw, two);
+                       0.5 * scale * scale, tw);
     MFIC_LAUNCH_CHECK();
 }
 

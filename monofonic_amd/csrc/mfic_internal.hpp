@@ -117,10 +117,11 @@ void* ctx_scratch(mfic_ctx ctx, const std::string& key, size_t bytes);
 // faults the device
 void require_device_memory(const void* p, const char* what);
 
-// twiddles: complex transform of length L (kind 0), or real rows of length
-// 2M (kind 1: complex length M table followed by M+1 untangle factors), or
-// the half-cell shift phases exp(i pi m / L), m < 2L (kind 2, FP64); the
-// inter-stage factors follow radix plan `variant` of the length
+// twiddles: complex transform of length L (kind 0; kind 3: in the order of
+// the transforms that read them from LDS), or real rows of length 2M (kind 1:
+// complex length M table followed by M+1 untangle factors), or the half-cell
+// shift phases exp(i pi m / L), m < 2L (kind 2, FP64); the inter-stage factors
+// follow radix plan `variant` of the length
 const void* twiddles(mfic_ctx ctx, int L, int kind, int prec, int variant = 0);
 // the radix plan selected for a pass (mfic_fft_pass) of length L: the default
 // of the pass unless mfic_fft_set_plan chose one
