@@ -50,10 +50,14 @@ k_pencils(Fields<T> f, long ps, long os, int tlen, T scale, const cx<T>* __restr
     // one address stepped along the pencil, so that none stays in registers
     const long off = (active ? outer * os + tg : 0) + q * ps, step = P * ps;
     const cx<T>* src = f.src[blockIdx.y] + off;
+    using Tw = PencilTw<T, L, V, P * TK>;
+    Tw tws;
+    tws.load(tw);
     cx<T> v[E];
 #pragma unroll
     for (int e = 0; e < E; ++e, src += step) v[e] = *src;
-    fft_pencil<T, L, FWD, V>(v, q, lds, LdsMap{t, tkp}, tw);
+    const cx<T>* ltw = tws.store(lds, L * tkp, tw);
+    fft_pencil<T, L, FWD, V, Tw::LDS>(v, q, lds, LdsMap{t, tkp}, ltw);
     if (active) {
         cx<T>* dst = f.dst[blockIdx.y] + off;
 #pragma unroll
@@ -392,15 +396,16 @@ static void launch_pencils_LV(mfic_ctx ctx, const Fields<T>& f, int count, long 
     int pad = 0;
     const auto ov = ctx->tiles.find(std::make_tuple(L, 0, prec_of<T>()));
     if (ov != ctx->tiles.end()) { tk = ov->second.first; pad = ov->second.second; }
-    while (tk > 4 && ((size_t)L * (tk + pad) * sizeof(T) > ctx->max_lds || P * tk > 1024)) tk /= 2;
+    using Tw = PencilTw<T, L, V, 64>;
+    while (tk > 4 && ((size_t)L * (tk + pad) * sizeof(T) + Tw::BYTES > ctx->max_lds || P * tk > 1024)) tk /= 2;
     if (tk < 4) tk = 4;  // tiles below 4 run as 4
     const int tkp = tk + pad;
-    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, 0, prec_of<T>(), V));
+    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, Tw::KIND, prec_of<T>(), V));
     const int gx = (tlen + tk - 1) / tk;
     const long ntiles = (long)gx * nouter;
     const bool xcd = nouter > 1;
     const dim3 grid((unsigned)(xcd ? xcd_grid(ntiles) : ntiles), count);
-    const size_t lds = (size_t)L * tkp * sizeof(T);
+    const size_t lds = (size_t)L * tkp * sizeof(T) + Tw::BYTES;
     ProfScope prof(ctx, "fft_pencils_L" + std::to_string(L) + (FWD ? "_fwd" : "_inv") + tag + (sizeof(T) == 8 ? "_f64" : "_f32"),
                    2.0 * (double)tlen * L * nouter * sizeof(cx<T>) * count);
     switch (tk) {

@@ -421,13 +421,13 @@ __device__ __forceinline__ void fft_stage(cx<T>* v, int q, cx<T>* lds, MAP m, co
 }
 
 // full transform of length L on registers v[E] (positions q + P e)
-template <typename T, int L, bool FWD, class MAP, class SYNC = BlockSync, bool SPLIT = false, int V = 0>
+template <typename T, int L, bool FWD, class MAP, class SYNC = BlockSync, bool SPLIT = false, int V = 0, bool TWR = false>
 __device__ __forceinline__ void fft_regs(cx<T>* v, int q, cx<T>* lds, MAP m, const cx<T>* __restrict__ tw) {
     constexpr int S = Plan<L, V>::S;
-    fft_stage<T, L, 0, FWD, MAP, SYNC, SPLIT, V>(v, q, lds, m, tw);
-    if constexpr (S > 1) fft_stage<T, L, 1 % S, FWD, MAP, SYNC, SPLIT, V>(v, q, lds, m, tw);
-    if constexpr (S > 2) fft_stage<T, L, 2 % S, FWD, MAP, SYNC, SPLIT, V>(v, q, lds, m, tw);
-    if constexpr (S > 3) fft_stage<T, L, 3 % S, FWD, MAP, SYNC, SPLIT, V>(v, q, lds, m, tw);
+    fft_stage<T, L, 0, FWD, MAP, SYNC, SPLIT, V, TWR>(v, q, lds, m, tw);
+    if constexpr (S > 1) fft_stage<T, L, 1 % S, FWD, MAP, SYNC, SPLIT, V, TWR>(v, q, lds, m, tw);
+    if constexpr (S > 2) fft_stage<T, L, 2 % S, FWD, MAP, SYNC, SPLIT, V, TWR>(v, q, lds, m, tw);
+    if constexpr (S > 3) fft_stage<T, L, 3 % S, FWD, MAP, SYNC, SPLIT, V, TWR>(v, q, lds, m, tw);
 }
 
 // Pencil passes (TK neighbouring columns per workgroup) exchange real and
@@ -436,10 +436,48 @@ __device__ __forceinline__ void fft_regs(cx<T>* v, int q, cx<T>* lds, MAP m, con
 // default LDS budget of a pencil tile: 128-byte row segments per pencil
 // position (16 complex FP32 columns) at 768 points, 32 at 512
 constexpr size_t PENCIL_LDS_CAP = 69632;
-template <typename T, int L, bool FWD, int V = 0>
+template <typename T, int L, bool FWD, int V = 0, bool TWR = false>
 __device__ __forceinline__ void fft_pencil(cx<T>* v, int q, cx<T>* lds, LdsMap m, const cx<T>* __restrict__ tw) {
-    fft_regs<T, L, FWD, LdsMap, BlockSync, true, V>(v, q, lds, m, tw);
+    fft_regs<T, L, FWD, LdsMap, BlockSync, true, V, TWR>(v, q, lds, m, tw);
 }
+
+// A plan's twiddles (TWR order) staged in LDS by the workgroup's threads:
+// load() early, store() before the first exchange, whose barrier publishes
+// them.
+template <typename T, int L, int V, int THREADS> struct TwStage {
+    static constexpr int SIZE = plan_tw_size<L, V>(), REGS = (SIZE + THREADS - 1) / THREADS;
+    cx<T> r[REGS > 0 ? REGS : 1];
+    __device__ __forceinline__ void load(const cx<T>* __restrict__ tw) {
+#pragma unroll
+        for (int i = 0; i < REGS; ++i)
+            if (i * THREADS + (int)threadIdx.x < SIZE) r[i] = tw[i * THREADS + threadIdx.x];
+    }
+    __device__ __forceinline__ const cx<T>* store(cx<T>* at) const {
+#pragma unroll
+        for (int i = 0; i < REGS; ++i)
+            if (i * THREADS + (int)threadIdx.x < SIZE) at[i * THREADS + threadIdx.x] = r[i];
+        return at;
+    }
+};
+// Twiddles of a pencil tile: in LDS for FP32, behind the exchange's `reals`
+// values.  A wavefront's 16-byte loads of them move 1 KB through the vector
+// cache whatever its lanes share, more than the data does; at 768 points FP32
+// the truncation passes go from 2.76 + 2.34 to 2.09 + 2.17 ms, at 384 the r2c
+// passes from 284 + 231 to 248 + 215 us.  FP64 tiles have half the lanes on
+// a factor and twice the LDS traffic: 288 points lose 3-9%, so they read memory.
+template <typename T, int L, int V, int THREADS> struct PencilTw : TwStage<T, L, V, THREADS> {
+    static constexpr bool LDS = sizeof(T) == 4;
+    static constexpr int KIND = LDS ? 3 : 0;  // of the table
+    static constexpr size_t BYTES = LDS ? plan_tw_size<L, V>() * sizeof(cx<T>) : 0;
+    using Base = TwStage<T, L, V, THREADS>;
+    __device__ __forceinline__ void load(const cx<T>* __restrict__ tw) {
+        if constexpr (LDS) Base::load(tw);
+    }
+    __device__ __forceinline__ const cx<T>* store(cx<T>* lds, int reals, const cx<T>* __restrict__ tw) const {
+        if constexpr (LDS) return Base::store(reinterpret_cast<cx<T>*>(reinterpret_cast<T*>(lds) + reals));
+        else return tw;
+    }
+};
 
 // Two transforms of the same length and positions (registers v and w) in
 // lockstep: each stage applies one set of twiddle loads to both, and the two

@@ -278,6 +278,9 @@ k_pencils_f(LD ld, ST st, long ncols, const cx<T>* __restrict__ tw, int xcd) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
     const int t = threadIdx.x % TK, q = threadIdx.x / TK, m = blockIdx.y;
+    using Tw = PencilTw<T, L, V, Plan<L, V>::P * TK>;
+    Tw tws;
+    tws.load(tw);
     const long col = (xcd ? xcd_tile(blockIdx.x, gridDim.x) : (long)blockIdx.x) * TK + t;
     const bool active = col < ncols;
     const long c = active ? col : 0;
@@ -290,7 +293,8 @@ k_pencils_f(LD ld, ST st, long ncols, const cx<T>* __restrict__ tw, int xcd) {
     for (int e = 0; e < E; ++e) v[e] = ld.template load<L, V>(lc, q, e);
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = ld.template fix<L, V>(lc, q, e, v[e]);
-    fft_pencil<T, L, FWD, V>(v, q, lds, LdsMap{t, TK}, tw);
+    const cx<T>* ltw = tws.store(lds, L * TK, tw);
+    fft_pencil<T, L, FWD, V, Tw::LDS>(v, q, lds, LdsMap{t, TK}, ltw);
     if (active) {
         const auto sc = st.template column<L>(c, m);
 #pragma unroll
@@ -325,6 +329,9 @@ k_hess_a(const cx<T>* __restrict__ f, StPadCol<T> st, long ncols, T kf, T scale,
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
     const int t = threadIdx.x % TK, q = threadIdx.x / TK;
+    using Tw = PencilTw<T, L, V, Plan<L, V>::P * TK>;
+    Tw tws;
+    tws.load(tw);
     const long col = (long)blockIdx.x * TK + t;
     const bool active = col < ncols;
     const cx<T>* src = f + (active ? col : 0);
@@ -338,6 +345,7 @@ k_hess_a(const cx<T>* __restrict__ f, StPadCol<T> st, long ncols, T kf, T scale,
         for (int e = 0; e < E; ++e) raw[e] = load(e);
     }
     const int top = gridDim.y == 1 ? 2 : 2 - (int)blockIdx.y, end = gridDim.y == 1 ? 0 : top;
+    const cx<T>* ltw = tws.store(lds, L * TK, tw);
 #pragma unroll 1
     for (int p = top; p >= end; --p) {
         cx<T> v[E];
@@ -352,7 +360,7 @@ k_hess_a(const cx<T>* __restrict__ f, StPadCol<T> st, long ncols, T kf, T scale,
             const cx<T> x = KEEP ? raw[KEEP ? e : 0] : v[e];
             v[e] = cx<T>{m * x.x, m * x.y};
         }
-        fft_pencil<T, L, false, V>(v, q, lds, LdsMap{t, TK}, tw);
+        fft_pencil<T, L, false, V, Tw::LDS>(v, q, lds, LdsMap{t, TK}, ltw);
         if (active) {
             const auto sc = st.template column<L>(col, p);
 #pragma unroll
@@ -372,6 +380,9 @@ k_hess_b(LdAx1<T, true> ld, StAx1<T, false> st, long ncols, T kf, const cx<T>* _
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
     const int t = threadIdx.x % TK, q = threadIdx.x / TK;
+    using Tw = PencilTw<T, L, V, Plan<L, V>::P * TK>;
+    Tw tws;
+    tws.load(tw);
     const long col = xcd_tile(blockIdx.x, gridDim.x) * TK + t;
     const bool active = col < ncols;
     const long c = active ? col : 0;
@@ -383,6 +394,7 @@ k_hess_b(LdAx1<T, true> ld, StAx1<T, false> st, long ncols, T kf, const cx<T>* _
 #pragma unroll
         for (int e = 0; e < E; ++e) raw[e] = ld.template load<L, V>(lc, q, e);
     }
+    const cx<T>* ltw = tws.store(lds, L * TK, tw);
 #pragma unroll 1
     for (int i = first; i < last; ++i) {
         const int pq = HessOrder::q(i), pr = HessOrder::r(i);
@@ -399,7 +411,7 @@ k_hess_b(LdAx1<T, true> ld, StAx1<T, false> st, long ncols, T kf, const cx<T>* _
             const cx<T> x = KEEP ? raw[KEEP ? e : 0] : v[e];
             v[e] = cx<T>{m * x.x, m * x.y};
         }
-        fft_pencil<T, L, false, V>(v, q, lds, LdsMap{t, TK}, tw);
+        fft_pencil<T, L, false, V, Tw::LDS>(v, q, lds, LdsMap{t, TK}, ltw);
         if (active) {
             const auto sc = st.template column<L>(c, HessOrder::slot(i));
 #pragma unroll
@@ -425,6 +437,9 @@ k_hess_bt(LdAx1<T, false> ld, StAx1<T, true> st, long ncols, T kf, const cx<T>* 
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
     const int t = threadIdx.x % TK, q = threadIdx.x / TK;
+    using Tw = PencilTw<T, L, V, Plan<L, V>::P * TK>;
+    Tw tws;
+    tws.load(tw);
     const long col = xcd_tile(blockIdx.x, gridDim.x) * TK + t;
     const bool active = col < ncols;
     const long c = active ? col : 0;
@@ -433,6 +448,7 @@ k_hess_bt(LdAx1<T, false> ld, StAx1<T, true> st, long ncols, T kf, const cx<T>* 
     cx<T> acc[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) acc[e] = cx<T>{0, 0};
+    const cx<T>* ltw = tws.store(lds, L * TK, tw);
 #pragma unroll 1
     for (int i = first; i < last; ++i) {
         const int pq = HessOrder::q(i), pr = HessOrder::r(i);
@@ -441,7 +457,7 @@ k_hess_bt(LdAx1<T, false> ld, StAx1<T, true> st, long ncols, T kf, const cx<T>* 
         cx<T> v[E];
 #pragma unroll
         for (int e = 0; e < E; ++e) v[e] = ld.template load<L, V>(lc, q, e);
-        fft_pencil<T, L, true, V>(v, q, lds, LdsMap{t, TK}, tw);
+        fft_pencil<T, L, true, V, Tw::LDS>(v, q, lds, LdsMap{t, TK}, ltw);
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const T g = G::template grad<T>(q, e, kf);  // band elements are not stored
@@ -471,19 +487,23 @@ k_hess_at(LdPadCol<T> ld, AdjointOut<T> o, long ncols, T kf, const cx<T>* __rest
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
     const int t = threadIdx.x % TK, q = threadIdx.x / TK;
+    using Tw = PencilTw<T, L, V, Plan<L, V>::P * TK>;
+    Tw tws;
+    tws.load(tw);
     const long col = (long)blockIdx.x * TK + t;
     const bool active = col < ncols;
     const long c = active ? col : 0;
     cx<T> acc[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) acc[e] = cx<T>{0, 0};
+    const cx<T>* ltw = tws.store(lds, L * TK, tw);
 #pragma unroll 1
     for (int p = 0; p < 3; ++p) {
         const auto lc = ld.template column<L>(c, p);
         cx<T> v[E];
 #pragma unroll
         for (int e = 0; e < E; ++e) v[e] = ld.template load<L, V>(lc, q, e);
-        fft_pencil<T, L, true, V>(v, q, lds, LdsMap{t, TK}, tw);
+        fft_pencil<T, L, true, V, Tw::LDS>(v, q, lds, LdsMap{t, TK}, ltw);
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const T g = G::template grad<T>(q, e, kf);
@@ -525,6 +545,9 @@ k_pencils_filter(LD ld, ST st, long ncols, const cx<T>* __restrict__ tw, int xcd
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
     const int t = threadIdx.x % TK, q = threadIdx.x / TK, m = blockIdx.y;
+    using Tw = PencilTw<T, L, V, Plan<L, V>::P * TK>;
+    Tw tws;
+    tws.load(tw);
     const long col = (xcd ? xcd_tile(blockIdx.x, gridDim.x) : (long)blockIdx.x) * TK + t;
     const bool active = col < ncols;
     const long c = active ? col : 0;
@@ -532,7 +555,8 @@ k_pencils_filter(LD ld, ST st, long ncols, const cx<T>* __restrict__ tw, int xcd
     cx<T> v[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = ld.template load<L, V>(lc, q, e);
-    fft_pencil<T, L, true, V>(v, q, lds, LdsMap{t, TK}, tw);
+    const cx<T>* ltw = tws.store(lds, L * TK, tw);
+    fft_pencil<T, L, true, V, Tw::LDS>(v, q, lds, LdsMap{t, TK}, ltw);
     const bool colzero = zero_kz_nyquist && (int)(c % G::KC) == G::NH;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -540,7 +564,11 @@ k_pencils_filter(LD ld, ST st, long ncols, const cx<T>* __restrict__ tw, int xcd
         const bool keep = !colzero && !G::band(q, e) && q + G::P * e != G::NH;
         v[e] = keep ? cscale(v[e], scale) : cx<T>{0, 0};
     }
-    fft_pencil<T, L, false, V>(v, q, lds, LdsMap{t, TK}, tw);
+    // a position of its own, so that the factors of the first transform do not
+    // stay in registers for the second
+    int q2 = q;
+    if constexpr (Tw::LDS) asm("" : "+v"(q2));
+    fft_pencil<T, L, false, V, Tw::LDS>(v, q2, lds, LdsMap{t, TK}, ltw);
     if (active) {
         const auto sc = st.template column<L>(c, m);
 #pragma unroll
@@ -572,6 +600,10 @@ static int pick_tile(mfic_ctx ctx, int pass, bool wide) {
     return tk < 4 ? 4 : tk;
 }
 
+template <typename T, int L, int V> constexpr size_t pencil_lds(int tk) {
+    return (size_t)L * tk * sizeof(T) + PencilTw<T, L, V, 64>::BYTES;
+}
+
 template <typename T> constexpr int prec_of() { return sizeof(T) == 8 ? MFIC_F64 : MFIC_F32; }
 template <typename T, int L> static std::string pass_name(const char* name) {
     return std::string(name) + "_L" + std::to_string(L) + (sizeof(T) == 8 ? "_f64" : "_f32");
@@ -592,8 +624,8 @@ static void launch_fv(mfic_ctx ctx, int pass, const LD& ld, const ST& st, long n
                       double bytes, bool xcd) {
     constexpr int P = Plan<L, V>::P;
     const int tk = pick_tile<T, L, V>(ctx, pass, true);
-    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, 0, prec_of<T>(), V));
-    const size_t lds = (size_t)L * tk * sizeof(T);
+    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, PencilTw<T, L, V, 64>::KIND, prec_of<T>(), V));
+    const size_t lds = pencil_lds<T, L, V>(tk);
     // axis-1 passes: 16-column tiles of rows with an odd pitch share cache
     // lines with their neighbours, which the XCD-aware order keeps in one L2
     const long ntiles = (ncols + tk - 1) / tk;
@@ -693,14 +725,14 @@ static void launch_hess(mfic_ctx ctx, const cx<T>* f, cx<T>* xb, T kf, T scale) 
     constexpr int P = Plan<L, V>::P, N = 2 * L / 3, kc = N / 2 + 1;
     constexpr bool KEEP = hess_keep<T, L, V>();
     const int tk = pick_tile<T, L, V>(ctx, MFIC_PASS_PAD_C2R_A, false);
-    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, 0, prec_of<T>(), V));
+    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, PencilTw<T, L, V, 64>::KIND, prec_of<T>(), V));
     const long cols = (long)N * kc;
     const long ntiles = (cols + tk - 1) / tk;
     const int members = ntiles >= 4096 ? 1 : 3;
     const dim3 grid((unsigned)ntiles, members);
     ProfScope prof(ctx, pass_name<T, L>("fft_c2rAh"), (double)cols * (members * N + 3 * L) * sizeof(cx<T>));
 #define CALL(K)                                                                                                \
-    hipLaunchKernelGGL((k_hess_a<T, L, K, V, KEEP>), grid, dim3(P * K), (size_t)L * K * sizeof(T), ctx->stream, \
+    hipLaunchKernelGGL((k_hess_a<T, L, K, V, KEEP>), grid, dim3(P * K), (pencil_lds<T, L, V>(K)), ctx->stream, \
                        f, StPadCol<T>{xb}, cols, kf, scale, tw);
     MFIC_TILE_SWITCH(P, CALL)
 #undef CALL
@@ -715,14 +747,14 @@ static void launch_hess_b(mfic_ctx ctx, const cx<T>* xb, cx<T>* out, T kf) {
     constexpr int P = Plan<L, V>::P, N = 2 * L / 3, kc = N / 2 + 1;
     constexpr bool KEEP = hess_keep<T, L, V>();
     const int tk = pick_tile<T, L, V>(ctx, MFIC_PASS_PAD_C2R_B, false);
-    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, 0, prec_of<T>(), V));
+    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, PencilTw<T, L, V, 64>::KIND, prec_of<T>(), V));
     const long cols = (long)L * kc;
     const long ntiles = (cols + tk - 1) / tk;
     const int members = ntiles * 3 >= 1024 ? 3 : 6;
     const dim3 grid((unsigned)xcd_grid(ntiles), members);
     ProfScope prof(ctx, pass_name<T, L>("fft_c2rBh"), (double)cols * (members * N + 6 * L) * sizeof(cx<T>));
 #define CALL(K)                                                                                                \
-    hipLaunchKernelGGL((k_hess_b<T, L, K, V, KEEP>), grid, dim3(P * K), (size_t)L * K * sizeof(T), ctx->stream, \
+    hipLaunchKernelGGL((k_hess_b<T, L, K, V, KEEP>), grid, dim3(P * K), (pencil_lds<T, L, V>(K)), ctx->stream, \
                        LdAx1<T, true>{xb}, StAx1<T, false>{out}, cols, kf, tw);
     MFIC_TILE_SWITCH(P, CALL)
 #undef CALL
@@ -749,12 +781,12 @@ template <typename T> void hessians_to_kbuf(mfic_ctx ctx, const void* f, size_t 
 template <typename T, int L, int V> static void launch_hess_bt(mfic_ctx ctx, const cx<T>* in, cx<T>* zb, T kf) {
     constexpr int P = Plan<L, V>::P, N = 2 * L / 3, kc = N / 2 + 1;
     const int tk = pick_tile<T, L, V>(ctx, MFIC_PASS_PAD_R2C_B, false);
-    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, 0, prec_of<T>(), V));
+    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, PencilTw<T, L, V, 64>::KIND, prec_of<T>(), V));
     const long cols = (long)L * kc;
     const dim3 grid((unsigned)xcd_grid((cols + tk - 1) / tk), 3);
     ProfScope prof(ctx, pass_name<T, L>("fft_r2cBt"), (double)cols * (6 * L + 3 * N) * sizeof(cx<T>));
 #define CALL(K)                                                                                                \
-    hipLaunchKernelGGL((k_hess_bt<T, L, K, V>), grid, dim3(P * K), (size_t)L * K * sizeof(T), ctx->stream,     \
+    hipLaunchKernelGGL((k_hess_bt<T, L, K, V>), grid, dim3(P * K), (pencil_lds<T, L, V>(K)), ctx->stream,     \
                        LdAx1<T, false>{in}, StAx1<T, true>{zb}, cols, kf, tw);
     MFIC_TILE_SWITCH(P, CALL)
 #undef CALL
@@ -764,12 +796,12 @@ template <typename T, int L, int V>
 static void launch_hess_at(mfic_ctx ctx, const cx<T>* zb, const AdjointOut<T>& o, T kf) {
     constexpr int P = Plan<L, V>::P, N = 2 * L / 3, kc = N / 2 + 1;
     const int tk = pick_tile<T, L, V>(ctx, MFIC_PASS_PAD_R2C_A, false);
-    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, 0, prec_of<T>(), V));
+    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, PencilTw<T, L, V, 64>::KIND, prec_of<T>(), V));
     const long cols = (long)N * kc;
     const dim3 grid((unsigned)((cols + tk - 1) / tk));
     ProfScope prof(ctx, pass_name<T, L>("fft_r2cAt"), (double)cols * (3 * L + 2 * N) * sizeof(cx<T>));
 #define CALL(K)                                                                                                \
-    hipLaunchKernelGGL((k_hess_at<T, L, K, V>), grid, dim3(P * K), (size_t)L * K * sizeof(T), ctx->stream,     \
+    hipLaunchKernelGGL((k_hess_at<T, L, K, V>), grid, dim3(P * K), (pencil_lds<T, L, V>(K)), ctx->stream,     \
                        LdPadCol<T>{zb}, o, cols, kf, tw);
     MFIC_TILE_SWITCH(P, CALL)
 #undef CALL
@@ -802,8 +834,8 @@ static void launch_filter_v(mfic_ctx ctx, int pass, const LD& ld, const ST& st, 
                             int zk, double scale, const char* name) {
     constexpr int P = Plan<L, V>::P;
     const int tk = pick_tile<T, L, V>(ctx, pass, true);
-    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, 0, prec_of<T>(), V));
-    const size_t lds = (size_t)L * tk * sizeof(T);
+    const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, PencilTw<T, L, V, 64>::KIND, prec_of<T>(), V));
+    const size_t lds = pencil_lds<T, L, V>(tk);
     const long ntiles = (ncols + tk - 1) / tk;
     const dim3 grid((unsigned)(xcd ? xcd_grid(ntiles) : ntiles), members);
     ProfScope prof(ctx, pass_name<T, L>(name), 2.0 * (double)ncols * L * sizeof(cx<T>) * members);
