@@ -103,8 +103,8 @@ SYMBOLS = [
     ("fused_src3_", "mfic::ProdSrc3>"),
     ("fused_src2q_", "mfic::ProdSrc2Q>"),
     ("fused_src2_", "mfic::ProdSrc2>"),
-    ("fft_c2rC_n", "k_rows_c2r_pruned<"),
-    ("fft_r2cC_n", "k_rows_r2c_prod<"),
+    ("fft_c2rAh_", "k_hess_a<"),
+    ("fft_c2rBh_", "k_hess_b<"),
     ("fft_c2rA_", "LdOperand<"),
     ("fft_c2rB_", "false, mfic::LdAx1<"),
     ("fft_r2cB_", "true, mfic::LdAx1<"),
@@ -125,8 +125,8 @@ def measured_traffic(name):
         return None
     prec = "double" if name.endswith("_f64") else "float"
     sym = next((s for p, s in SYMBOLS if name.startswith(p)), None)
-    if sym is None or name.startswith("fft_r2cC_n"):
-        return None  # product-row launches of every width share one kernel symbol
+    if sym is None:
+        return None
     hits = []
     for line in open(TRAFFIC_FILE):
         if line.startswith("#") or not line.strip():

@@ -121,8 +121,8 @@ int mfic_fft_size_supported(size_t n);
  * pass that also forms the shifted sub-lattice; rows per block for kind 1
  * contiguous-axis passes; kinds 3..8, the padded convolver pass kinds of
  * mfic_fft_pass below, override kind 0 for that pass only) and the LDS pitch
- * padding (kinds 0 and 1) for one transform length and precision; tile <= 0
- * restores the built-in choice.  No reference counterpart (FFTW planning,
+ * padding (kinds 0 and 1) for one transform length and precision; strided
+ * tiles below 4 run as 4; tile <= 0 restores the built-in choice.  No reference counterpart (FFTW planning,
  * grid_fft.cc:53-54, plays this role there). */
 int mfic_fft_set_tile(mfic_ctx ctx, int length, int kind, int prec, int tile, int lds_pad);
 /* the override of mfic_fft_set_tile for a key (tile 0: the built-in choice) */
@@ -131,8 +131,9 @@ int mfic_fft_get_tile(mfic_ctx ctx, int length, int kind, int prec, int *tile, i
 /* Radix plans.  Each transform length has a compiled default plan (elements
  * per thread and the radix of each Stockham stage); the padded-pass lengths
  * 512 and 768 also have an alternative with twice the elements per thread
- * and 16 threads per transform.  A strided pass of one kind selects its plan
- * per length and precision (the row passes keep their own plans); the fused
+ * and 16 threads per transform, the default of the 768-point FP32 truncation
+ * filters.  A strided pass of one kind selects its plan per length and
+ * precision (the row passes keep their own plans); the fused
  * source row passes select one of two forms the same way.  No reference
  * counterpart: FFTW picks its codelets while planning (grid_fft.cc:53-54). */
 enum mfic_fft_pass {
@@ -234,8 +235,8 @@ typedef struct {
     int kind;        /* mfic_opkind                               */
     int d[4];        /* directions (HESS: d0 d1; SUM/DIFF: d0..d3) */
 } mfic_operand;
-/* OrszagConvolver<real_t>(N, L) (convolution.hh:446-478): owns the two
- * padded 3N/2 grids and the N-grid buffer. */
+/* OrszagConvolver<real_t>(N, L) (convolution.hh:446-478): owns its padded
+ * intermediates, compact half-spectra of 3N/2 x 3N/2 x (N/2 + 1) values. */
 typedef struct mfic_conv_s *mfic_conv;
 int mfic_conv_create(mfic_ctx ctx, const size_t n[3], const double L[3], int prec, mfic_conv *out);
 int mfic_conv_destroy(mfic_conv c);
