@@ -425,8 +425,8 @@ k_hess_b(LdAx1<T, true> ld, StAx1<T, false> st, long ncols, T kf, const cx<T>* _
 // factors separate per axis, so pass B' sums the fields of an x power after
 // their axis-1 transforms, weighted by -g_j^q g_k^r, and pass A' the three
 // sums after theirs, weighted by g_i^p: three axis-0 transforms and one write
-// of the result for six of each.  Bound by memory: at 256^3 FP32 pass B' 291 us
-// (4.2 TB/s) for six fields, pass A' 160 us (2.8 TB/s; 16 columns to a tile,
+// of the result for six of each.  Bound by memory: at 256^3 FP32 pass B' 274 us
+// (4.4 TB/s) for six fields, pass A' 160 us (2.8 TB/s; 16 columns to a tile,
 // whose factors and table reads are FP64), where one field took 63 + 45 us and
 // 58 us for its weighted sum.
 template <typename T, int L, int TK, int V>
