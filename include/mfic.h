@@ -236,7 +236,9 @@ typedef struct {
     int d[4];        /* directions (HESS: d0 d1; SUM/DIFF: d0..d3) */
 } mfic_operand;
 /* OrszagConvolver<real_t>(N, L) (convolution.hh:446-478): owns its padded
- * intermediates, compact half-spectra of 3N/2 x 3N/2 x (N/2 + 1) values. */
+ * intermediates, compact half-spectra of 3N/2 x 3N/2 x (N/2 + 1) values.
+ * One size on every axis (MFIC_ERR_SIZE otherwise); operands and outputs have
+ * the convolver's size and precision (MFIC_ERR_ARG). */
 typedef struct mfic_conv_s *mfic_conv;
 int mfic_conv_create(mfic_ctx ctx, const size_t n[3], const double L[3], int prec, mfic_conv *out);
 int mfic_conv_destroy(mfic_conv c);

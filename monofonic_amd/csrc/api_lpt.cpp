@@ -58,8 +58,18 @@ static void need(mfic_grid g, const char* what) {
     MFIC_CHECK(g && g->d, MFIC_ERR_ARG, std::string("null or unallocated grid: ") + what);
 }
 
-static OperandDesc to_desc(const mfic_operand* o) {
+// grids that one pass reads or writes with the strides of another
+static void need_like(mfic_grid g, mfic_grid ref, const char* what) {
+    need(g, what);
+    MFIC_CHECK(g->prec == ref->prec && g->n[0] == ref->n[0] && g->n[1] == ref->n[1] && g->n[2] == ref->n[2],
+               MFIC_ERR_ARG, std::string("grid size or precision differs from phi1's: ") + what);
+}
+
+static OperandDesc to_desc(const mfic_operand* o, const ConvCore& c) {
     MFIC_CHECK(o && o->f && o->f->d, MFIC_ERR_ARG, "null operand");
+    MFIC_CHECK(o->f->prec == c.prec, MFIC_ERR_ARG, "precision mismatch");
+    MFIC_CHECK(o->f->n[0] == c.N[0] && o->f->n[1] == c.N[1] && o->f->n[2] == c.N[2], MFIC_ERR_ARG,
+               "operand grid does not match the convolver");
     MFIC_CHECK(o->kind >= MFIC_OPND_HESS && o->kind <= MFIC_OPND_IDENT, MFIC_ERR_ARG, "bad operand kind");
     for (int i = 0; i < 4; ++i) MFIC_CHECK(o->d[i] >= 0 && o->d[i] < 3, MFIC_ERR_ARG, "operand direction out of range");
     MFIC_CHECK(o->f->space == MFIC_KSPACE, MFIC_ERR_STATE, "operand fields must be in k-space");
@@ -210,8 +220,7 @@ int mfic_conv_convolve2(mfic_conv c, const mfic_operand* a, const mfic_operand* 
     return guard_call([&] {
         conv_check_out(c, out);
         MFIC_CHECK(op >= MFIC_OP_ASSIGN && op <= MFIC_OP_MADD, MFIC_ERR_ARG, "bad output operator");
-        const OperandDesc da = to_desc(a), db = to_desc(b);
-        MFIC_CHECK(a->f->prec == c->core->prec && b->f->prec == c->core->prec, MFIC_ERR_ARG, "precision mismatch");
+        const OperandDesc da = to_desc(a, *c->core), db = to_desc(b, *c->core);
         c->core->convolve2(da, db, out->d, op, coef, c->kbuf);
         out->space = MFIC_KSPACE;
     });
@@ -222,7 +231,7 @@ int mfic_conv_convolve3(mfic_conv c, const mfic_operand* a, const mfic_operand* 
     return guard_call([&] {
         conv_check_out(c, out);
         MFIC_CHECK(op >= MFIC_OP_ASSIGN && op <= MFIC_OP_MADD, MFIC_ERR_ARG, "bad output operator");
-        const OperandDesc da = to_desc(a), db = to_desc(b), dc = to_desc(cc);
+        const OperandDesc da = to_desc(a, *c->core), db = to_desc(b, *c->core), dc = to_desc(cc, *c->core);
         c->core->convolve3(da, db, dc, out->d, op, coef, c->kbuf, c->fbuf);
         out->space = MFIC_KSPACE;
     });
@@ -235,8 +244,11 @@ int mfic_lpt_sources(mfic_ctx ctx, int order, mfic_grid phi1, mfic_grid phi2, mf
         MFIC_CHECK(order >= 1 && order <= 3, MFIC_ERR_CONFIG, "LPT order must be 1, 2 or 3");
         need(phi1, "phi1");
         MFIC_CHECK(phi1->space == MFIC_KSPACE, MFIC_ERR_STATE, "phi1 must be in k-space");
-        if (order > 1) need(phi2, "phi2");
-        if (order > 2) { need(phi3, "phi3"); need(A3x, "A3x"); need(A3y, "A3y"); need(A3z, "A3z"); }
+        if (order > 1) need_like(phi2, phi1, "phi2");
+        if (order > 2) {
+            need_like(phi3, phi1, "phi3");
+            need_like(A3x, phi1, "A3x"); need_like(A3y, phi1, "A3y"); need_like(A3z, phi1, "A3z");
+        }
         lpt_sources(ctx, order, phi1, phi2, phi3, A3x, A3y, A3z);
     });
 }
@@ -288,12 +300,12 @@ int mfic_lpt_component(mfic_ctx ctx, int order, int comp, const mfic_lpt_coef* k
         MFIC_CHECK(comp >= 0 && comp < 6, MFIC_ERR_ARG, "component must be 0..5");
         MFIC_CHECK(order >= 1 && order <= 3, MFIC_ERR_CONFIG, "LPT order must be 1, 2 or 3");
         need(phi1, "phi1");
-        need(out, "out");
-        const void* phi[3] = {phi1->d, order > 1 ? (need(phi2, "phi2"), phi2->d) : nullptr,
-                              order > 2 ? (need(phi3, "phi3"), phi3->d) : nullptr};
+        need_like(out, phi1, "out");
+        const void* phi[3] = {phi1->d, order > 1 ? (need_like(phi2, phi1, "phi2"), phi2->d) : nullptr,
+                              order > 2 ? (need_like(phi3, phi1, "phi3"), phi3->d) : nullptr};
         const void* A3[3] = {nullptr, nullptr, nullptr};
         if (order > 2) {
-            need(A3x, "A3x"); need(A3y, "A3y"); need(A3z, "A3z");
+            need_like(A3x, phi1, "A3x"); need_like(A3y, phi1, "A3y"); need_like(A3z, phi1, "A3z");
             A3[0] = A3x->d; A3[1] = A3y->d; A3[2] = A3z->d;
         }
         double cf[4];

@@ -23,6 +23,8 @@
 namespace mfic {
 
 ConvCore::ConvCore(mfic_ctx c, const size_t n[3], const double L[3], int p) : ctx(c), prec(p) {
+    // the passes take every stride and column count from one size
+    MFIC_CHECK(n[0] == n[1] && n[1] == n[2], MFIC_ERR_SIZE, "the Orszag convolver needs the same grid size on every axis");
     for (int i = 0; i < 3; ++i) {
         MFIC_CHECK(n[i] % 2 == 0, MFIC_ERR_SIZE, "Orszag convolver for LPTorder>1 requires even grid size!");
         N[i] = n[i];
@@ -66,7 +68,6 @@ void lpt_sources(mfic_ctx ctx, int order, mfic_grid phi1, mfic_grid phi2, mfic_g
                  mfic_grid A3y, mfic_grid A3z) {
     if (order < 2) return;
     ConvCore C(ctx, phi1->n, phi1->L, phi1->prec);
-    MFIC_CHECK(phi1->n[0] == phi1->n[1] && phi1->n[1] == phi1->n[2], MFIC_ERR_SIZE, "LPT sources need a cubic grid");
     const size_t n = phi1->n[0];
     const double L = phi1->L[0];
     const int prec = phi1->prec;
