@@ -237,8 +237,8 @@ typedef struct {
 } mfic_operand;
 /* OrszagConvolver<real_t>(N, L) (convolution.hh:446-478): owns its padded
  * intermediates, compact half-spectra of 3N/2 x 3N/2 x (N/2 + 1) values.
- * One size on every axis (MFIC_ERR_SIZE otherwise); operands and outputs have
- * the convolver's size and precision (MFIC_ERR_ARG). */
+ * One size on every axis (MFIC_ERR_SIZE otherwise), any sides L; operands and
+ * outputs have the convolver's size and precision (MFIC_ERR_ARG). */
 typedef struct mfic_conv_s *mfic_conv;
 int mfic_conv_create(mfic_ctx ctx, const size_t n[3], const double L[3], int prec, mfic_conv *out);
 int mfic_conv_destroy(mfic_conv c);
@@ -260,7 +260,8 @@ int mfic_conv_convolve3(mfic_conv c, const mfic_operand *a, const mfic_operand *
  * per order forms every product sharing a truncation (FP64 sums) in LDS and
  * returns r2c'd rows, the cubic terms keep their two-stage truncation.
  * Growth factors are NOT applied here (mfic_lpt_component applies them).
- * Grids not needed for the order may be NULL. */
+ * Grids not needed for the order may be NULL; the others have phi1's size and
+ * precision (MFIC_ERR_ARG), and the box is a cube (MFIC_ERR_SIZE). */
 int mfic_lpt_sources(mfic_ctx ctx, int order, mfic_grid phi1, mfic_grid phi2, mfic_grid phi3,
                      mfic_grid A3x, mfic_grid A3y, mfic_grid A3z);
 
@@ -287,7 +288,8 @@ int mfic_plt_download(mfic_plt p, double *Dr, double *Dtheta, double *Dphi, doub
  * Growth factors g1..g3c and vfac1..3 are applied here in FP64 (the
  * reference applies them to the potentials at ic_generator.cc:644-658,
  * which is the same product).  plt may be NULL (Fourier gradient,
- * operators.hh:38-61).  out is left in k-space. */
+ * operators.hh:38-61).  The grids have one size and precision (MFIC_ERR_ARG)
+ * in a cubic box (MFIC_ERR_SIZE).  out is left in k-space. */
 int mfic_lpt_component(mfic_ctx ctx, int order, int comp, const mfic_lpt_coef *k, mfic_plt plt,
                        double unit, mfic_grid phi1, mfic_grid phi2, mfic_grid phi3, mfic_grid A3x,
                        mfic_grid A3y, mfic_grid A3z, mfic_grid out);

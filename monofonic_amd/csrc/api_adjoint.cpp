@@ -210,7 +210,7 @@ int mfic_lpt2_adjoint(mfic_lpt2 p, mfic_grid noise, mfic_grid cot_x, mfic_grid c
         char* ws = static_cast<char*>(mfic::ctx_scratch(p->ctx, "lpt2_adjoint", 13 * kb));
         mfic::padded_hessians_to_kbuf(p->ctx, p->prec, p->phi1.g->d, p->n, p->L, ws + 7 * kb, ws);
         const mfic::OperandDesc lmu{p->lmu.g->d, MFIC_OPND_IDENT, {0, 0, 0, 0}};
-        mfic::padded_operands_to_kbuf(p->ctx, p->prec, &lmu, 1, p->n, p->L, ws + 6 * kb);
+        mfic::padded_operands_to_kbuf(p->ctx, p->prec, &lmu, 1, p->n, p->core->len, ws + 6 * kb);
         mfic::fused_source_rows(p->ctx, p->prec, mfic::FusedKind::Adjoint2, p->n, ws, ws + 7 * kb);
         // phi1 branch and the adjoint of phi1 = S P_N r2c(noise)
         mfic::padded_hessian_adjoint(p->ctx, p->prec, p->n, p->L, ws + 7 * kb, ws, p->lam.g->d,

@@ -313,6 +313,7 @@ int mfic_lpt_component(mfic_ctx ctx, int order, int comp, const mfic_lpt_coef* k
         PltDev pv;
         if (plt) pv = plt->t.view;
         MFIC_CHECK(phi1->n[0] == phi1->n[1] && phi1->n[1] == phi1->n[2], MFIC_ERR_SIZE, "assembly needs a cubic grid");
+        MFIC_CHECK(out->L[0] == out->L[1] && out->L[1] == out->L[2], MFIC_ERR_SIZE, "assembly needs equal box sides");
         assemble_component(ctx, out->prec, out->n, out->L[0], order, comp, cf, unit, pv, phi, A3, out->d, nullptr);
         out->space = MFIC_KSPACE;
     });

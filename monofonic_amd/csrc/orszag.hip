@@ -50,7 +50,7 @@ void ConvCore::convolve2(const OperandDesc& a, const OperandDesc& b, void* out, 
     const bool square = a.same(b);
     const OperandDesc o[2] = {a, b};
     void* prod = static_cast<char*>(kbuf) + 2 * kbuf_reals() * esize();
-    padded_operands_to_kbuf(ctx, prec, o, square ? 1 : 2, N[0], len[0], kbuf);
+    padded_operands_to_kbuf(ctx, prec, o, square ? 1 : 2, N[0], len, kbuf);
     fused_source_rows(ctx, prec, square ? FusedKind::Square : FusedKind::Mul, N[0], kbuf, prod);
     padded_r2c_from_kbuf(ctx, prec, N[0], len[0], prod, 1, &out, op, coef, false);
 }
@@ -68,6 +68,7 @@ void lpt_sources(mfic_ctx ctx, int order, mfic_grid phi1, mfic_grid phi2, mfic_g
                  mfic_grid A3y, mfic_grid A3z) {
     if (order < 2) return;
     ConvCore C(ctx, phi1->n, phi1->L, phi1->prec);
+    MFIC_CHECK(phi1->L[0] == phi1->L[1] && phi1->L[1] == phi1->L[2], MFIC_ERR_SIZE, "LPT sources need equal box sides");
     const size_t n = phi1->n[0];
     const double L = phi1->L[0];
     const int prec = phi1->prec;

@@ -91,7 +91,7 @@ template <typename T> __device__ __forceinline__ T grad_t(int idx, int n, T kf) 
 template <typename T> struct LdOperand {
     struct Op { const cx<T>* f; int kind, d0, d1, d2, d3; };
     Op op[2];
-    double kf, scale;
+    double kf[3], scale;  // 2 pi / L of each axis
     struct Col { const cx<T>* p; double al, be, ga; bool imag; };
     // product -(g_a g_b) as polynomial coefficients in g_i
     __device__ __forceinline__ static void prod2(int a, int b, double gj, double gk, double sg, double& al, double& be,
@@ -109,7 +109,7 @@ template <typename T> struct LdOperand {
         const Op o = op[m];
         const int d0 = o.d0, d1 = o.d1, d2 = o.d2, d3 = o.d3;
         c.p = o.f + col;
-        const double gj = grad_t<double>(j, G::N, kf), gk = grad_t<double>(k, G::N, kf);
+        const double gj = grad_t<double>(j, G::N, kf[1]), gk = grad_t<double>(k, G::N, kf[2]);
         c.al = c.be = c.ga = 0.0;
         c.imag = false;
         switch (o.kind) {
@@ -141,7 +141,7 @@ template <typename T> struct LdOperand {
     template <int L, int V = 0> __device__ __forceinline__ cx<T> fix(const Col& c, int q, int e, cx<T> v) const {
         using G = PadGeo<L, V>;
         if (G::band(q, e)) return v;
-        const double g = G::template grad<double>(q, e, kf);
+        const double g = G::template grad<double>(q, e, kf[0]);
         const double s = (c.al * g + c.be) * g + c.ga;
         return c.imag ? cx<T>{(T)(-s * (double)v.y), (T)(s * (double)v.x)}
                       : cx<T>{(T)(s * (double)v.x), (T)(s * (double)v.y)};
@@ -660,12 +660,12 @@ static void launch_f(mfic_ctx ctx, int pass, const LD& ld, const ST& st, long nc
     }
 
 template <typename T>
-void operands_to_kbuf(mfic_ctx ctx, const OperandDesc* o, int count, size_t n, double L, void* kbuf) {
+void operands_to_kbuf(mfic_ctx ctx, const OperandDesc* o, int count, size_t n, const double L[3], void* kbuf) {
     const int N = (int)n, np = 3 * N / 2, kc = N / 2 + 1;
     LdOperand<T> la{};
     for (int m = 0; m < count; ++m)
         la.op[m] = {static_cast<const cx<T>*>(o[m].f), o[m].kind, o[m].d[0], o[m].d[1], o[m].d[2], o[m].d[3]};
-    la.kf = 2.0 * 3.14159265358979323846 / L;
+    for (int a = 0; a < 3; ++a) la.kf[a] = 2.0 * 3.14159265358979323846 / L[a];
     la.scale = std::pow(1.5, 1.5);
     StPadCol<T> sa{static_cast<cx<T>*>(kbuf)};
     LdAx1<T, true> lb{static_cast<const cx<T>*>(kbuf)};
@@ -875,7 +875,7 @@ template <typename T> void truncate_repad(mfic_ctx ctx, size_t n, void* kbuf, in
 }
 
 #define MFIC_PRUNED_T(MODE, T)                                                                                        \
-    MODE template void operands_to_kbuf<T>(mfic_ctx, const OperandDesc*, int, size_t, double, void*);                 \
+    MODE template void operands_to_kbuf<T>(mfic_ctx, const OperandDesc*, int, size_t, const double*, void*);                \
     MODE template void r2c_from_kbuf<T>(mfic_ctx, size_t, double, void*, int, void* const*, int, double, bool);       \
     MODE template void hessians_to_kbuf<T>(mfic_ctx, const void*, size_t, double, void*, void*);                      \
     MODE template void hessian_adjoint<T>(mfic_ctx, size_t, double, const void*, void*, const void*, const double*,   \
@@ -903,7 +903,8 @@ void padded_truncate_repad(mfic_ctx ctx, int prec, size_t n, void* kbuf, int cou
     else truncate_repad<float>(ctx, n, kbuf, count);
 }
 
-void padded_operands_to_kbuf(mfic_ctx ctx, int prec, const OperandDesc* o, int count, size_t n, double L, void* kbuf) {
+void padded_operands_to_kbuf(mfic_ctx ctx, int prec, const OperandDesc* o, int count, size_t n, const double L[3],
+                             void* kbuf) {
     MFIC_CHECK(count == 1 || count == 2, MFIC_ERR_ARG, "one or two operands");
     if (prec == MFIC_F64) operands_to_kbuf<double>(ctx, o, count, n, L, kbuf);
     else operands_to_kbuf<float>(ctx, o, count, n, L, kbuf);

@@ -7,8 +7,10 @@ namespace mfic {
 
 // operands of N-grid k-space fields -> consecutive compact padded buffers
 // ([Np][Np][N/2+1] complex each) after the axis-0 and axis-1 c2r passes
-// (half-spectrum rows ready for a row pass); one or two operands
-void padded_operands_to_kbuf(mfic_ctx ctx, int prec, const OperandDesc* o, int count, size_t n, double L, void* kbuf);
+// (half-spectrum rows ready for a row pass) in a box of sides L; one or two
+// operands
+void padded_operands_to_kbuf(mfic_ctx ctx, int prec, const OperandDesc* o, int count, size_t n, const double L[3],
+                             void* kbuf);
 // the six Hessians xx yy zz xy xz yz of an N-grid k-space field -> six
 // consecutive compact padded buffers (out) after the axis-0 and axis-1 c2r
 // passes; xbuf is scratch for three compact buffers
