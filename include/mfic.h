@@ -365,7 +365,9 @@ int mfic_run_potential(mfic_run r, int which, mfic_grid *out);
  * by mfic_graph_launch.  Whatever the captured calls allocate lazily (scratch
  * buffers, twiddle tables) must already exist: execute the same sequence once
  * before capturing.  A call that would allocate fails with MFIC_ERR_STATE and
- * mfic_graph_end then reports the broken capture.  Per-kernel timing is
+ * mfic_graph_end then reports the broken capture.  A graph may be replayed
+ * after larger boxes have run on the context: scratch that it uses is kept
+ * when it is outgrown and freed with the last graph.  Per-kernel timing is
  * suspended while capturing. */
 typedef struct mfic_graph_s *mfic_graph;
 int mfic_graph_begin(mfic_ctx ctx);

@@ -34,17 +34,28 @@ template <typename F> static int guard(F&& f) {
 
 void* ctx_scratch(mfic_ctx ctx, const std::string& key, size_t bytes) {
     auto& s = ctx->scratch[key];
-    if (s.second < bytes) {
+    if (s.bytes < bytes) {
         MFIC_CHECK(!ctx->capturing, MFIC_ERR_STATE,
                    "scratch '" + key + "' would grow during graph capture: run the sequence once before capturing");
-        if (s.first) MFIC_HIP(hipFree(s.first));
-        s.first = nullptr;
-        s.second = 0;
-        hipError_t e = hipMalloc(&s.first, bytes);
-        if (e != hipSuccess) throw Error(MFIC_ERR_ALLOC, "scratch allocation of " + std::to_string(bytes) + " bytes failed");
-        s.second = bytes;
+        if (s.captured && ctx->graphs > 0) ctx->retired.push_back(s.p);  // a graph's launches hold its address
+        else if (s.p) MFIC_HIP(hipFree(s.p));
+        s = mfic_scratch{};
+        hipError_t e = hipMalloc(&s.p, bytes);
+        if (e != hipSuccess) {
+            s.p = nullptr;
+            throw Error(MFIC_ERR_ALLOC, "scratch allocation of " + std::to_string(bytes) + " bytes failed");
+        }
+        s.bytes = bytes;
     }
-    return s.first;
+    if (ctx->capturing) s.captured = true;
+    return s.p;
+}
+
+void ctx_graph_destroyed(mfic_ctx ctx) {
+    if (--ctx->graphs > 0 || ctx->capturing) return;
+    for (void* p : ctx->retired) (void)hipFree(p);
+    ctx->retired.clear();
+    for (auto& kv : ctx->scratch) kv.second.captured = false;
 }
 
 static hipEvent_t pool_event(mfic_ctx ctx) {
@@ -137,7 +148,8 @@ int mfic_ctx_destroy(mfic_ctx ctx) {
         (void)hipSetDevice(ctx->device);
         (void)hipStreamSynchronize(ctx->stream);
         for (auto& kv : ctx->tables) (void)hipFree(kv.second.dev);
-        for (auto& kv : ctx->scratch) (void)hipFree(kv.second.first);
+        for (auto& kv : ctx->scratch) (void)hipFree(kv.second.p);
+        for (void* p : ctx->retired) (void)hipFree(p);
         for (auto& r : ctx->prof_recs) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
         for (auto& e : ctx->prof_pool) (void)hipEventDestroy(e);
         (void)hipStreamDestroy(ctx->stream);

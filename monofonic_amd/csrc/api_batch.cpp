@@ -47,6 +47,7 @@ int mfic_graph_end(mfic_ctx ctx, mfic_graph* out) {
             throw mfic::Error(MFIC_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(ei));
         }
         ++ctx->children;
+        ++ctx->graphs;
         *out = r;
     });
 }
@@ -68,6 +69,7 @@ int mfic_graph_destroy(mfic_graph g) {
         if (g->graph) (void)hipGraphDestroy(g->graph);
         mfic_ctx ctx = g->ctx;
         delete g;
+        mfic::ctx_graph_destroyed(ctx);
         --ctx->children;
     });
 }

@@ -53,6 +53,13 @@ struct mfic_prof_rec {
     hipEvent_t a, b;
 };
 
+// a scratch buffer of a context; captured: its address may be in a live graph
+struct mfic_scratch {
+    void* p = nullptr;
+    size_t bytes = 0;
+    bool captured = false;
+};
+
 struct mfic_ctx_s {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -60,7 +67,11 @@ struct mfic_ctx_s {
     std::map<std::tuple<int, int, int>, mfic::TwTable> tables;
     std::mutex mu;
     // scratch buffers owned by the context (reused across calls)
-    std::map<std::string, std::pair<void*, size_t>> scratch;
+    std::map<std::string, mfic_scratch> scratch;
+    // graphs alive, and the buffers they use that have been outgrown since:
+    // those stay allocated until the last graph is destroyed
+    long graphs = 0;
+    std::vector<void*> retired;
     size_t max_lds = 0;  // LDS bytes per workgroup (device attribute)
     // tile overrides from the autotuner: (length, kind, prec) -> (tile, lds pad)
     std::map<std::tuple<int, int, int>, std::pair<int, int>> tiles;
@@ -109,8 +120,11 @@ class ProfScope {
     long idx_ = -1;
 };
 
-// scratch buffer of at least `bytes`, keyed by name, owned by the context
+// scratch buffer of at least `bytes`, keyed by name, owned by the context.  A
+// buffer that grows moves; the old one is freed unless a live graph uses it.
 void* ctx_scratch(mfic_ctx ctx, const std::string& key, size_t bytes);
+// a graph of the context is gone (its stream synchronised)
+void ctx_graph_destroyed(mfic_ctx ctx);
 
 // refuses (MFIC_ERR_ARG) a caller pointer that kernels would access but that
 // is not device or managed memory: a kernel store to pageable host memory
