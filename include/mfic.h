@@ -400,7 +400,9 @@ int mfic_autotune_config(mfic_ctx ctx, const mfic_ic_config *cfg, const mfic_cos
  * mfic_lpt2_adjoint maps cotangents of Psi_x, Psi_y, Psi_z back to the
  * gradient with respect to delta (reverse mode, hand-written), recomputing
  * phi1 from delta instead of storing forward intermediates.  All grids are
- * real-space n^3 grids of the plan's precision. */
+ * real-space n^3 grids of the plan's precision.  The plan owns seven n^3 grids
+ * and thirteen half-spectra of 3n/2 x 3n/2 x (n/2 + 1) values (16 GB at 512^3
+ * FP32), allocated in create (MFIC_ERR_ALLOC) and freed in destroy. */
 typedef struct mfic_lpt2_s *mfic_lpt2;
 int mfic_lpt2_create(mfic_ctx ctx, size_t n, double L, int prec, const mfic_cosmo_params *cosmo, double unit,
                      mfic_lpt2 *out);

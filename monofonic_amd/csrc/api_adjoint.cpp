@@ -44,13 +44,19 @@ struct mfic_lpt2_s {
     mfic_lpt_coef coef{};
     GridPtr phi1, phi2, lam, lmu, t[3];
     std::unique_ptr<mfic::ConvCore> core;  // sizes of the padded passes
+    void* ws = nullptr;    // compact padded buffers of the adjoint
     void* d_tk = nullptr;  // spline nodes of a tabulated transfer function
     ~mfic_lpt2_s() {
+        if (ws) (void)hipFree(ws);
         if (d_tk) (void)hipFree(d_tk);
     }
 };
 
 namespace {
+// compact padded buffers: Hessians of phi1 [0, 6), lam_mu [6], the six products
+// [7, 13); the x powers pass through [7, 10) on the way in and [0, 3) on the
+// way out
+constexpr size_t WS_BUFFERS = 13;
 void make(mfic_lpt2_s* p, GridPtr& g, int space) {
     const size_t n3[3] = {p->n, p->n, p->n};
     const double L3[3] = {p->L, p->L, p->L};
@@ -146,6 +152,12 @@ int mfic_lpt2_create(mfic_ctx ctx, size_t n, double L, int prec, const mfic_cosm
         const size_t n3[3] = {n, n, n};
         const double L3[3] = {L, L, L};
         p->core = std::make_unique<mfic::ConvCore>(ctx, n3, L3, prec);
+        const size_t wsb = WS_BUFFERS * p->core->kbuf_reals() * p->core->esize();
+        if (hipMalloc(&p->ws, wsb) != hipSuccess) {
+            (void)hipGetLastError();
+            p->ws = nullptr;
+            throw Error(MFIC_ERR_ALLOC, "2LPT plan: workspace allocation of " + std::to_string(wsb) + " bytes failed");
+        }
         ++ctx->children;
         *out = p.release();
     });
@@ -203,11 +215,8 @@ int mfic_lpt2_adjoint(mfic_lpt2 p, mfic_grid noise, mfic_grid cot_x, mfic_grid c
         // lam = unit sum_d (-i g_d) G_d (adjoint of the gradient, unit and
         // DC := 0) and lam_mu = P_N lap^-1 (g2 lam) of the phi2 branch
         mfic::kspace_grad_adjoint(p->lam.g, p->lmu.g, t[0], t[1], t[2], p->unit, p->coef.g2);
-        // compact padded buffers: Hessians of phi1 [0, 6), lam_mu [6], the
-        // six products [7, 13); the x powers pass through [7, 10) on the way
-        // in and [0, 3) on the way out
         const size_t kb = p->core->kbuf_reals() * p->core->esize();
-        char* ws = static_cast<char*>(mfic::ctx_scratch(p->ctx, "lpt2_adjoint", 13 * kb));
+        char* ws = static_cast<char*>(p->ws);
         mfic::padded_hessians_to_kbuf(p->ctx, p->prec, p->phi1.g->d, p->n, p->L, ws + 7 * kb, ws);
         const mfic::OperandDesc lmu{p->lmu.g->d, MFIC_OPND_IDENT, {0, 0, 0, 0}};
         mfic::padded_operands_to_kbuf(p->ctx, p->prec, &lmu, 1, p->n, p->core->len, ws + 6 * kb);

@@ -1,16 +1,18 @@
 """Work spaces that a captured graph uses stay where they are while a later,
 larger box outgrows them: replays give the bits of the eager run, and the
-outgrown buffers are given back with the last graph."""
+outgrown buffers are given back with the last graph.  The 2LPT adjoint works in
+a space of its plan."""
 import ctypes as C
 
 import numpy as np
 import pytest
 
-from monofonic_amd import F32, F64, Context, lpt
+from monofonic_amd import F32, F64, Context, Grid, lpt
 from monofonic_amd.batch import capture
 from monofonic_amd.lpt import ICConfig, ICRun
 
 torch = pytest.importorskip("torch")
+from monofonic_amd.adjoint import LPT2  # noqa: E402
 
 
 def free_bytes():
@@ -92,5 +94,61 @@ def test_growth_without_a_graph_keeps_nothing():
         grown = 23 * (kb(128) - kb(96))
         print(f"96^3 -> 128^3: {at96 - at128} bytes more, {grown} expected")
         assert at96 - at128 <= grown + (16 << 20)  # tables and allocation granules
+    finally:
+        ctx.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,n,larger", [(F32, 32, 96), (F64, 48, 64)])
+def test_adjoint_replay_after_a_larger_plan(prec, n, larger):
+    ctx = Context(0)
+    try:
+        rng = np.random.default_rng(n)
+        dtype = np.float64 if prec == F64 else np.float32
+        plan = LPT2(ctx, n, 100.0, prec=prec)
+        grids = [Grid(ctx, (n,) * 3, (100.0,) * 3, prec=prec) for _ in range(5)]
+        for g in grids[:4]:
+            g.upload(rng.standard_normal(g.shape_real).astype(dtype))
+        adjoint = lambda: plan.adjoint_grids(grids[0], grids[1:4], grids[4])  # noqa: E731
+        adjoint()
+        want = grids[4].download_r().copy()
+        graph = capture(ctx, adjoint)
+        big = LPT2(ctx, larger, 100.0, prec=prec)
+        x = torch.randn(larger, larger, larger, dtype=torch.float64, device="cuda")
+        big.adjoint(x, torch.stack([x, -x, 2 * x]))
+        for rep in range(3):
+            grids[4].zero()
+            graph.launch()
+            assert np.array_equal(grids[4].download_r(), want), rep
+            if rep == 0:
+                big.close()
+        graph.close()
+        for o in (plan, *grids):
+            o.close()
+    finally:
+        ctx.close()
+
+
+@pytest.mark.gpu
+def test_a_plan_owns_its_workspace():
+    """taken when the plan is made, not at the first adjoint, and given back
+    with the plan"""
+    ctx = Context(0)
+    try:
+        n, prec = 128, F32
+        x = torch.randn(n, n, n, device="cuda")
+        cot = torch.stack([x, x, x])
+        first = LPT2(ctx, n, 100.0, prec=prec)  # allocates what the context keeps
+        first.forward(x), first.adjoint(x, cot)
+        first.close()
+        before = free_bytes()
+        plan = LPT2(ctx, n, 100.0, prec=prec)
+        made = free_bytes()
+        workspace = 13 * (3 * n // 2) ** 2 * (n // 2 + 1) * 8
+        assert before - made >= workspace
+        plan.adjoint(x, cot)
+        assert made - free_bytes() <= 2 << 20
+        plan.close()
+        assert before - free_bytes() <= 2 << 20
     finally:
         ctx.close()
