@@ -430,7 +430,8 @@ int mfic_fft_c2c(mfic_ctx ctx, void *data, const size_t n[3], int prec, int forw
  * v_d = D+ vfac / L * velocity_unit * hbar Im(psi* d_d psi) / (1 + delta)
  * with d_d = i k_d in k-space (get_k, Nyquist at +n/2).  The run's species
  * is dark matter without baryons (C_species = 0, so sqrt(rho) = 1).  Outputs
- * are real-space grids of the run's size and precision; hbar may be NULL. */
+ * are real-space grids of the run's size and precision; hbar may be NULL.  The
+ * first call takes work arrays of four such grids, which the run keeps. */
 int mfic_ppt_fields(mfic_run r, double velocity_unit, mfic_grid delta, mfic_grid vx, mfic_grid vy, mfic_grid vz,
                     double *hbar);
 

@@ -46,6 +46,7 @@ struct mfic_run_s {
     double *d_pos = nullptr, *d_vel = nullptr;
     double *d_pos_b = nullptr, *d_vel_b = nullptr;  // baryon species (secondary lattice)
     size_t npart = 0;
+    void* ppt_ws = nullptr;  // work arrays of mfic_ppt_fields, made by its first call
     mfic::PltTables plt;
     bool has_plt = false;
     ~mfic_run_s();
@@ -160,6 +161,7 @@ mfic_run_s::~mfic_run_s() {
     if (d_vel) (void)hipFree(d_vel);
     if (d_pos_b) (void)hipFree(d_pos_b);
     if (d_vel_b) (void)hipFree(d_vel_b);
+    if (ppt_ws) (void)hipFree(ppt_ws);
 }
 
 extern "C" {
@@ -708,10 +710,11 @@ int mfic_ppt_fields(mfic_run r, double velocity_unit, mfic_grid delta, mfic_grid
         const size_t n = c.n, es = c.prec == MFIC_F64 ? 8 : 4;
         const size_t nn[3] = {n, n, n};
         const double norm = 1.0 / std::sqrt((double)n * n * n);
-        // growth-scaled real-space potentials (ic_generator.cc:644-658, 809, 847)
-        // and psi, in a workspace of the context
+        MFIC_CHECK(!r->ctx->capturing, MFIC_ERR_STATE, "PPT fields synchronise (hbar): they cannot be captured");
+        // the two potentials in real space and psi
         const size_t greal = n * n * (n + 2) * es, slot = (greal + 255) / 256 * 256;
-        char* ws = static_cast<char*>(ctx_scratch(r->ctx, "ppt_work", 2 * slot + n * n * n * 2 * es));
+        if (!r->ppt_ws) r->ppt_ws = dmalloc(2 * slot + n * n * n * 2 * es, "PPT work arrays");
+        char* ws = static_cast<char*>(r->ppt_ws);
         void* ph1 = ws;
         void* ph2 = c.lpt_order >= 2 ? ws + slot : nullptr;
         // growth-scaled real-space potentials (ic_generator.cc:644-658, 809, 847)
