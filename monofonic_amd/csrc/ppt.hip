@@ -359,13 +359,19 @@ static void ppt_passes(mfic_ctx ctx, const PptInput& in, double hbar, T* delta, 
                            vel[2], rows, inv, kn, vh, tw);
         MFIC_LAUNCH_CHECK();
     }
+    // a buffer given for several components ends up with the last of them, z
+    // (written above) before y before x
     ProfScope prof(ctx, "ppt_pencil_velocity" + tag, 2.0 * n3 * (sizeof(cx<T>) + sizeof(T)));
-    hipLaunchKernelGGL((k_ppt_pencil_velocity<T, L, TK, 0>), pgrid, dim3(P * TK), plds, ctx->stream, psi, vel[0], kn,
-                       vh, tw);
-    MFIC_LAUNCH_CHECK();
-    hipLaunchKernelGGL((k_ppt_pencil_velocity<T, L, TK, 1>), dim3((unsigned)xcd_grid(pgrid.x)), dim3(P * TK), plds,
-                       ctx->stream, psi, vel[1], kn, vh, tw);
-    MFIC_LAUNCH_CHECK();
+    if (vel[0] != vel[2]) {
+        hipLaunchKernelGGL((k_ppt_pencil_velocity<T, L, TK, 0>), pgrid, dim3(P * TK), plds, ctx->stream, psi, vel[0],
+                           kn, vh, tw);
+        MFIC_LAUNCH_CHECK();
+    }
+    if (vel[1] != vel[2]) {
+        hipLaunchKernelGGL((k_ppt_pencil_velocity<T, L, TK, 1>), dim3((unsigned)xcd_grid(pgrid.x)), dim3(P * TK), plds,
+                           ctx->stream, psi, vel[1], kn, vh, tw);
+        MFIC_LAUNCH_CHECK();
+    }
 }
 
 template <typename T>

@@ -64,3 +64,23 @@ def test_fields_are_refused_under_capture(ctx):
         assert np.array_equal(a.download_r(), b)
     for o in (graph, *outs, *again, run):
         o.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("same", [(0, 1), (0, 2), (1, 2), (0, 1, 2)])
+def test_one_grid_for_several_velocities(ctx, same):
+    """holds the last of its components, as passes in the order x, y, z leave it"""
+    n = 24
+    run = lpt.ICRun(ctx, lpt.ICConfig(n=n, box=50.0, zstart=24.0, lpt_order=2, prec=F64, seed=3))
+    run.execute()
+    want, _ = lpt.ppt_fields(run)
+    ref = [g.download_r().copy() for g in want]
+    outs = [Grid(ctx, (n,) * 3, (50.0,) * 3, prec=F64) for _ in range(4)]
+    vel = [outs[1 + (same[0] if d in same else d)] for d in range(3)]
+    L.call("mfic_ppt_fields", run.h, 1.0, outs[0].h, *[g.h for g in vel], None)
+    assert np.array_equal(outs[0].download_r(), ref[0])
+    for d in range(3):
+        last = same[-1] if d in same else d
+        assert np.array_equal(vel[d].download_r(), ref[1 + last]), d
+    for o in (*want, *outs, run):
+        o.close()
