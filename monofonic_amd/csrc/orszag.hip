@@ -99,6 +99,14 @@ void lpt_sources(mfic_ctx ctx, int order, mfic_grid phi1, mfic_grid phi2, mfic_g
     char* kout = static_cast<char*>(ctx_scratch(ctx, "fused_out", 4 * kb));
     fused_source_rows(ctx, prec, FusedKind::Src3, n, kin, kout);
     void* outs[4] = {phi3->d, A3x->d, A3y->d, A3z->d};
+    // one launch writes them all: a grid given several times takes the last,
+    // the others go to the x powers' buffers, whose work is done
+    for (int o = 0; o < 3; ++o)
+        for (int e = o + 1; e < 4; ++e)
+            if (outs[o] == outs[e]) {
+                outs[o] = static_cast<char*>(xbuf) + o * kb;
+                break;
+            }
     padded_r2c_from_kbuf(ctx, prec, n, L, kout, 4, outs, MFIC_OP_ASSIGN, 0.0, true);
     for (mfic_grid g : {phi3, A3x, A3y, A3z}) g->space = MFIC_KSPACE;
 }

@@ -142,3 +142,23 @@ def test_unequal_sides_of_a_potential_are_refused(ctx, sides):
                   out.h) == ERR_SIZE
     for x in (*g, out):
         x.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,n", [(F64, 32), (F32, 96)])
+@pytest.mark.parametrize("same", [(0, 1), (1, 2, 3), (0, 3), (0, 1, 2, 3)])
+def test_one_grid_for_several_potentials(ctx, same, prec, n):
+    """of phi3, A3x, A3y, A3z given the same grid, it holds the last"""
+    g = [k_grid(ctx, n, prec) for _ in range(6)]
+    lpt.ngenic_fill(g[0], 4)
+    lpt.lpt_sources(ctx, 3, g[0], g[1], g[2], g[3:])
+    want = [x.download_k().copy() for x in g[2:]]
+    out = [g[2 + (same[0] if i in same else i)] for i in range(4)]
+    for rep in range(3):
+        for x in g[1:]:
+            x.zero()
+        lpt.lpt_sources(ctx, 3, g[0], g[1], out[0], out[1:])
+        for i in range(4):
+            assert np.array_equal(out[i].download_k(), want[same[-1] if i in same else i]), (rep, i)
+    for x in g:
+        x.close()
