@@ -120,9 +120,11 @@ int mfic_fft_size_supported(size_t n);
  * strided pass of the length, and for kind 2, the bcc particle path's axis-0
  * pass that also forms the shifted sub-lattice; rows per block for kind 1
  * contiguous-axis passes; kinds 3..8, the padded convolver pass kinds of
- * mfic_fft_pass below, override kind 0 for that pass only) and the LDS pitch
- * padding (kinds 0 and 1) for one transform length and precision; strided
- * tiles below 4 run as 4; tile <= 0 restores the built-in choice.  No reference counterpart (FFTW planning,
+ * mfic_fft_pass below, override kind 0 for that pass only) for one transform
+ * length and precision; strided tiles below 4 run as 4; tile <= 0 restores
+ * the built-in choice.  lds_pad, 0 to 8 pencils added to the LDS pitch, is
+ * honoured by the N-grid strided passes (kind 0 at their length); every other
+ * pass keeps its own pitch.  No reference counterpart (FFTW planning,
  * grid_fft.cc:53-54, plays this role there). */
 int mfic_fft_set_tile(mfic_ctx ctx, int length, int kind, int prec, int tile, int lds_pad);
 /* the override of mfic_fft_set_tile for a key (tile 0: the built-in choice) */

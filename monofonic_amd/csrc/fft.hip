@@ -397,7 +397,7 @@ static void launch_pencils_LV(mfic_ctx ctx, const Fields<T>& f, int count, long 
     const auto ov = ctx->tiles.find(std::make_tuple(L, 0, prec_of<T>()));
     if (ov != ctx->tiles.end()) { tk = ov->second.first; pad = ov->second.second; }
     using Tw = PencilTw<T, L, V, 64>;
-    while (tk > 4 && ((size_t)L * (tk + pad) * sizeof(T) + Tw::BYTES > ctx->max_lds || P * tk > 1024)) tk /= 2;
+    while (tk > 4 && (Tw::bytes((size_t)L * (tk + pad)) > ctx->max_lds || P * tk > 1024)) tk /= 2;
     if (tk < 4) tk = 4;  // tiles below 4 run as 4
     const int tkp = tk + pad;
     const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, Tw::KIND, prec_of<T>(), V));
@@ -405,7 +405,7 @@ static void launch_pencils_LV(mfic_ctx ctx, const Fields<T>& f, int count, long 
     const long ntiles = (long)gx * nouter;
     const bool xcd = nouter > 1;
     const dim3 grid((unsigned)(xcd ? xcd_grid(ntiles) : ntiles), count);
-    const size_t lds = (size_t)L * tkp * sizeof(T) + Tw::BYTES;
+    const size_t lds = Tw::bytes((size_t)L * tkp);
     ProfScope prof(ctx, "fft_pencils_L" + std::to_string(L) + (FWD ? "_fwd" : "_inv") + tag + (sizeof(T) == 8 ? "_f64" : "_f32"),
                    2.0 * (double)tlen * L * nouter * sizeof(cx<T>) * count);
     switch (tk) {

@@ -468,13 +468,19 @@ template <typename T, int L, int V, int THREADS> struct TwStage {
 template <typename T, int L, int V, int THREADS> struct PencilTw : TwStage<T, L, V, THREADS> {
     static constexpr bool LDS = sizeof(T) == 4;
     static constexpr int KIND = LDS ? 3 : 0;  // of the table
-    static constexpr size_t BYTES = LDS ? plan_tw_size<L, V>() * sizeof(cx<T>) : 0;
     using Base = TwStage<T, L, V, THREADS>;
+    // first real of the table behind an exchange of `reals`: complex values sit
+    // at even ones (an odd length on an odd pitch makes `reals` odd)
+    static __host__ __device__ constexpr size_t table_at(size_t reals) { return reals + (LDS ? reals % 2 : 0); }
+    // LDS of the exchange and the table
+    static constexpr size_t bytes(size_t reals) {
+        return table_at(reals) * sizeof(T) + (LDS ? plan_tw_size<L, V>() * sizeof(cx<T>) : 0);
+    }
     __device__ __forceinline__ void load(const cx<T>* __restrict__ tw) {
         if constexpr (LDS) Base::load(tw);
     }
     __device__ __forceinline__ const cx<T>* store(cx<T>* lds, int reals, const cx<T>* __restrict__ tw) const {
-        if constexpr (LDS) return Base::store(reinterpret_cast<cx<T>*>(reinterpret_cast<T*>(lds) + reals));
+        if constexpr (LDS) return Base::store(reinterpret_cast<cx<T>*>(reinterpret_cast<T*>(lds) + table_at(reals)));
         else return tw;
     }
 };

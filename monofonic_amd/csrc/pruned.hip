@@ -601,7 +601,7 @@ static int pick_tile(mfic_ctx ctx, int pass, bool wide) {
 }
 
 template <typename T, int L, int V> constexpr size_t pencil_lds(int tk) {
-    return (size_t)L * tk * sizeof(T) + PencilTw<T, L, V, 64>::BYTES;
+    return PencilTw<T, L, V, 64>::bytes((size_t)L * tk);
 }
 
 template <typename T> constexpr int prec_of() { return sizeof(T) == 8 ? MFIC_F64 : MFIC_F32; }
