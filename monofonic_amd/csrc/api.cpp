@@ -394,7 +394,8 @@ int mfic_fft_set_tile(mfic_ctx ctx, int length, int kind, int prec, int tile, in
         if (tile <= 0) { ctx->tiles.erase(key); return; }
         MFIC_CHECK((tile & (tile - 1)) == 0 && tile <= 64, MFIC_ERR_ARG, "tile must be a power of two <= 64");
         MFIC_CHECK(lds_pad >= 0 && lds_pad <= 8, MFIC_ERR_ARG, "lds_pad must be in [0, 8]");
-        ctx->tiles[key] = {tile, lds_pad};
+        // strided passes are built for tiles of 4 and more
+        ctx->tiles[key] = {kind != 1 && tile < 4 ? 4 : tile, lds_pad};
     });
 }
 

@@ -2,6 +2,8 @@
 exchange and the twiddles behind it, not the arithmetic, so every override
 gives the bits of the built-in choice.  9 is the one odd length: with an odd
 pad its exchange has an odd number of reals."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -39,3 +41,16 @@ def test_pads_change_nothing(ctx, shape, prec):
     finally:
         for n in lengths:
             L.call("mfic_fft_set_tile", ctx.h, n, 0, prec, 0, 0)
+
+
+@pytest.mark.gpu
+def test_reported_tiles_are_those_that_run(ctx):
+    t, pad = C.c_int(), C.c_int()
+    for length, kind in ((64, 0), (64, 1), (64, 2), (96, L.PASS_PAD_C2R_A), (96, L.PASS_TRUNC_AX1)):
+        try:
+            for tile in (1, 2, 4, 16):
+                L.call("mfic_fft_set_tile", ctx.h, length, kind, F32, tile, 0)
+                L.call("mfic_fft_get_tile", ctx.h, length, kind, F32, C.byref(t), C.byref(pad))
+                assert t.value == (tile if kind == 1 else max(tile, 4)), (length, kind, tile)
+        finally:
+            L.call("mfic_fft_set_tile", ctx.h, length, kind, F32, 0, 0)
