@@ -217,7 +217,7 @@ int mfic_lpt2_adjoint(mfic_lpt2 p, mfic_grid noise, mfic_grid cot_x, mfic_grid c
         mfic::kspace_grad_adjoint(p->lam.g, p->lmu.g, t[0], t[1], t[2], p->unit, p->coef.g2);
         const size_t kb = p->core->kbuf_reals() * p->core->esize();
         char* ws = static_cast<char*>(p->ws);
-        mfic::padded_hessians_to_kbuf(p->ctx, p->prec, p->phi1.g->d, p->n, p->L, ws + 7 * kb, ws);
+        mfic::padded_hessians_to_kbuf(p->ctx, p->prec, p->phi1.g->d, p->n, p->L, ws + 7 * kb, ws, true);
         const mfic::OperandDesc lmu{p->lmu.g->d, MFIC_OPND_IDENT, {0, 0, 0, 0}};
         mfic::padded_operands_to_kbuf(p->ctx, p->prec, &lmu, 1, p->n, p->core->len, ws + 6 * kb);
         mfic::fused_source_rows(p->ctx, p->prec, mfic::FusedKind::Adjoint2, p->n, ws, ws + 7 * kb);

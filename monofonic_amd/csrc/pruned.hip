@@ -320,10 +320,12 @@ struct HessOrder {
 
 // A workgroup reads a tile of source pencils once and makes the outputs of
 // all x powers (gridDim.y = 1) or one (3).  KEEP holds the pencil in
-// registers for the next power; else it is read again, from cache.
-template <typename T, int L, int TK, int V, bool KEEP>
+// registers for the next power; else it is read again, from cache.  The weights
+// are formed and applied in W: T for the LPT sources, FP64 for the 2LPT adjoint
+// (256^3 FP32: pass A 110 us against 98, pass B 314 against 313).
+template <typename T, typename W, int L, int TK, int V, bool KEEP>
 __global__ void __launch_bounds__((Plan<L, V>::P * TK))
-k_hess_a(const cx<T>* __restrict__ f, StPadCol<T> st, long ncols, T kf, T scale, const cx<T>* __restrict__ tw) {
+k_hess_a(const cx<T>* __restrict__ f, StPadCol<T> st, long ncols, W kf, W scale, const cx<T>* __restrict__ tw) {
     using G = PadGeo<L, V>;
     constexpr int E = Plan<L, V>::E;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -355,10 +357,10 @@ k_hess_a(const cx<T>* __restrict__ f, StPadCol<T> st, long ncols, T kf, T scale,
         }
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const T g = G::template grad<T>(q, e, kf);
-            const T m = scale * (p > 0 ? g : T(1)) * (p > 1 ? g : T(1));
+            const W g = G::template grad<W>(q, e, kf);
+            const W m = scale * (p > 0 ? g : W(1)) * (p > 1 ? g : W(1));
             const cx<T> x = KEEP ? raw[KEEP ? e : 0] : v[e];
-            v[e] = cx<T>{m * x.x, m * x.y};
+            v[e] = cx<T>{(T)(m * x.x), (T)(m * x.y)};
         }
         fft_pencil<T, L, false, V, Tw::LDS>(v, q, lds, LdsMap{t, TK}, ltw);
         if (active) {
@@ -372,9 +374,9 @@ k_hess_a(const cx<T>* __restrict__ f, StPadCol<T> st, long ncols, T kf, T scale,
 // Pass B: g_j^q along the pencil (zero band skipped) times the per-column
 // factor -g_k^r; gridDim.y = 3 reads the pencils of an x power once for all
 // its Hessians, 6 takes each Hessian by itself.
-template <typename T, int L, int TK, int V, bool KEEP>
+template <typename T, typename W, int L, int TK, int V, bool KEEP>
 __global__ void __launch_bounds__((Plan<L, V>::P * TK))
-k_hess_b(LdAx1<T, true> ld, StAx1<T, false> st, long ncols, T kf, const cx<T>* __restrict__ tw) {
+k_hess_b(LdAx1<T, true> ld, StAx1<T, false> st, long ncols, W kf, const cx<T>* __restrict__ tw) {
     using G = PadGeo<L, V>;
     constexpr int E = Plan<L, V>::E;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -388,7 +390,7 @@ k_hess_b(LdAx1<T, true> ld, StAx1<T, false> st, long ncols, T kf, const cx<T>* _
     const long c = active ? col : 0;
     const int first = HessOrder::first(blockIdx.y, gridDim.y), last = HessOrder::last(blockIdx.y, gridDim.y);
     const auto lc = ld.template column<L>(c, HessOrder::p(first));
-    const T gk = grad_t<T>((int)(c % G::KC), G::N, kf);
+    const W gk = grad_t<W>((int)(c % G::KC), G::N, kf);
     cx<T> raw[KEEP ? E : 1];
     if constexpr (KEEP) {
 #pragma unroll
@@ -398,7 +400,7 @@ k_hess_b(LdAx1<T, true> ld, StAx1<T, false> st, long ncols, T kf, const cx<T>* _
 #pragma unroll 1
     for (int i = first; i < last; ++i) {
         const int pq = HessOrder::q(i), pr = HessOrder::r(i);
-        const T cm = pr == 0 ? T(-1) : (pr == 1 ? T(-1) * gk : T(-1) * (gk * gk));
+        const W cm = pr == 0 ? W(-1) : (pr == 1 ? W(-1) * gk : W(-1) * (gk * gk));
         cx<T> v[E];
         if constexpr (!KEEP) {
 #pragma unroll
@@ -406,10 +408,10 @@ k_hess_b(LdAx1<T, true> ld, StAx1<T, false> st, long ncols, T kf, const cx<T>* _
         }
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const T g = G::template grad<T>(q, e, kf);
-            const T m = cm * (pq > 0 ? g : T(1)) * (pq > 1 ? g : T(1));
+            const W g = G::template grad<W>(q, e, kf);
+            const W m = cm * (pq > 0 ? g : W(1)) * (pq > 1 ? g : W(1));
             const cx<T> x = KEEP ? raw[KEEP ? e : 0] : v[e];
-            v[e] = cx<T>{m * x.x, m * x.y};
+            v[e] = cx<T>{(T)(m * x.x), (T)(m * x.y)};
         }
         fft_pencil<T, L, false, V, Tw::LDS>(v, q, lds, LdsMap{t, TK}, ltw);
         if (active) {
@@ -425,13 +427,15 @@ k_hess_b(LdAx1<T, true> ld, StAx1<T, false> st, long ncols, T kf, const cx<T>* _
 // factors separate per axis, so pass B' sums the fields of an x power after
 // their axis-1 transforms, weighted by -g_j^q g_k^r, and pass A' the three
 // sums after theirs, weighted by g_i^p: three axis-0 transforms and one write
-// of the result for six of each.  Bound by memory: at 256^3 FP32 pass B' 274 us
-// (4.4 TB/s) for six fields, pass A' 160 us (2.8 TB/s; 16 columns to a tile,
-// whose factors and table reads are FP64), where one field took 63 + 45 us and
-// 58 us for its weighted sum.
+// of the result for six of each.  Weights and multiply-adds are FP64, the sums
+// are rounded to T at each addition, as sums kept in memory field by field
+// would be (FP64 sums put pass B' on one wave a SIMD: forward and adjoint 3.74
+// ms against 3.57).  Bound by memory: at 256^3 FP32 pass B' 270 us (4.5 TB/s)
+// for six fields, pass A' 159 us (2.8 TB/s; 16 columns to a tile), where one
+// field took 63 + 45 us and 58 us for its weighted sum.
 template <typename T, int L, int TK, int V>
 __global__ void __launch_bounds__((Plan<L, V>::P * TK))
-k_hess_bt(LdAx1<T, false> ld, StAx1<T, true> st, long ncols, T kf, const cx<T>* __restrict__ tw) {
+k_hess_bt(LdAx1<T, false> ld, StAx1<T, true> st, long ncols, double kf, const cx<T>* __restrict__ tw) {
     using G = PadGeo<L, V>;
     constexpr int E = Plan<L, V>::E;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -444,7 +448,7 @@ k_hess_bt(LdAx1<T, false> ld, StAx1<T, true> st, long ncols, T kf, const cx<T>* 
     const bool active = col < ncols;
     const long c = active ? col : 0;
     const int first = HessOrder::first(blockIdx.y, 3), last = HessOrder::last(blockIdx.y, 3);
-    const T gk = grad_t<T>((int)(c % G::KC), G::N, kf);
+    const double gk = grad_t<double>((int)(c % G::KC), G::N, kf);
     cx<T> acc[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) acc[e] = cx<T>{0, 0};
@@ -452,7 +456,7 @@ k_hess_bt(LdAx1<T, false> ld, StAx1<T, true> st, long ncols, T kf, const cx<T>* 
 #pragma unroll 1
     for (int i = first; i < last; ++i) {
         const int pq = HessOrder::q(i), pr = HessOrder::r(i);
-        const T cm = pr == 0 ? T(-1) : (pr == 1 ? T(-1) * gk : T(-1) * (gk * gk));
+        const double cm = pr == 0 ? -1.0 : (pr == 1 ? -gk : -(gk * gk));
         const auto lc = ld.template column<L>(c, HessOrder::slot(i));
         cx<T> v[E];
 #pragma unroll
@@ -460,9 +464,9 @@ k_hess_bt(LdAx1<T, false> ld, StAx1<T, true> st, long ncols, T kf, const cx<T>* 
         fft_pencil<T, L, true, V, Tw::LDS>(v, q, lds, LdsMap{t, TK}, ltw);
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const T g = G::template grad<T>(q, e, kf);  // band elements are not stored
-            const T m = cm * (pq > 0 ? g : T(1)) * (pq > 1 ? g : T(1));
-            acc[e] = cx<T>{acc[e].x + m * v[e].x, acc[e].y + m * v[e].y};
+            const double g = G::template grad<double>(q, e, kf);  // band elements are not stored
+            const double m = cm * (pq > 0 ? g : 1.0) * (pq > 1 ? g : 1.0);
+            acc[e] = cx<T>{(T)(acc[e].x + m * v[e].x), (T)(acc[e].y + m * v[e].y)};
         }
     }
     if (active) {
@@ -481,7 +485,7 @@ template <typename T> struct AdjointOut {
 };
 template <typename T, int L, int TK, int V>
 __global__ void __launch_bounds__((Plan<L, V>::P * TK))
-k_hess_at(LdPadCol<T> ld, AdjointOut<T> o, long ncols, T kf, const cx<T>* __restrict__ tw) {
+k_hess_at(LdPadCol<T> ld, AdjointOut<T> o, long ncols, double kf, const cx<T>* __restrict__ tw) {
     using G = PadGeo<L, V>;
     constexpr int E = Plan<L, V>::E;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -506,9 +510,9 @@ k_hess_at(LdPadCol<T> ld, AdjointOut<T> o, long ncols, T kf, const cx<T>* __rest
         fft_pencil<T, L, true, V, Tw::LDS>(v, q, lds, LdsMap{t, TK}, ltw);
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const T g = G::template grad<T>(q, e, kf);
-            const T m = (p > 0 ? g : T(1)) * (p > 1 ? g : T(1));
-            acc[e] = cx<T>{acc[e].x + m * v[e].x, acc[e].y + m * v[e].y};
+            const double g = G::template grad<double>(q, e, kf);
+            const double m = (p > 0 ? g : 1.0) * (p > 1 ? g : 1.0);
+            acc[e] = cx<T>{(T)(acc[e].x + m * v[e].x), (T)(acc[e].y + m * v[e].y)};
         }
     }
     if (!active) return;
@@ -720,8 +724,8 @@ template <typename T, int L, int V> constexpr bool hess_keep() { return Plan<L, 
 // tiles to fill the chip several times over, else a power each (pass A of
 // 512^3 FP32: 0.77 ms as one member, 1.01 as three, 1.84 as three launches
 // that read the field each time; 64^3 FP64 8.3, 5.8 and 24 us).
-template <typename T, int L, int V>
-static void launch_hess(mfic_ctx ctx, const cx<T>* f, cx<T>* xb, T kf, T scale) {
+template <typename T, typename W, int L, int V>
+static void launch_hess(mfic_ctx ctx, const cx<T>* f, cx<T>* xb, W kf, W scale) {
     constexpr int P = Plan<L, V>::P, N = 2 * L / 3, kc = N / 2 + 1;
     constexpr bool KEEP = hess_keep<T, L, V>();
     const int tk = pick_tile<T, L, V>(ctx, MFIC_PASS_PAD_C2R_A, false);
@@ -732,7 +736,7 @@ static void launch_hess(mfic_ctx ctx, const cx<T>* f, cx<T>* xb, T kf, T scale) 
     const dim3 grid((unsigned)ntiles, members);
     ProfScope prof(ctx, pass_name<T, L>("fft_c2rAh"), (double)cols * (members * N + 3 * L) * sizeof(cx<T>));
 #define CALL(K)                                                                                                \
-    hipLaunchKernelGGL((k_hess_a<T, L, K, V, KEEP>), grid, dim3(P * K), (pencil_lds<T, L, V>(K)), ctx->stream, \
+    hipLaunchKernelGGL((k_hess_a<T, W, L, K, V, KEEP>), grid, dim3(P * K), (pencil_lds<T, L, V>(K)), ctx->stream, \
                        f, StPadCol<T>{xb}, cols, kf, scale, tw);
     MFIC_TILE_SWITCH(P, CALL)
 #undef CALL
@@ -742,8 +746,8 @@ static void launch_hess(mfic_ctx ctx, const cx<T>* f, cx<T>* xb, T kf, T scale) 
 // workgroups a CU on, below that a member per Hessian (512^3 FP32: 2.68 ms
 // against 3.06 as six members and 3.5 as six launches on the same plan;
 // 256^3 FP32 317, 394 and 380 us; 64^3 FP32 9.4, 7.8 and 26 us).
-template <typename T, int L, int V>
-static void launch_hess_b(mfic_ctx ctx, const cx<T>* xb, cx<T>* out, T kf) {
+template <typename T, typename W, int L, int V>
+static void launch_hess_b(mfic_ctx ctx, const cx<T>* xb, cx<T>* out, W kf) {
     constexpr int P = Plan<L, V>::P, N = 2 * L / 3, kc = N / 2 + 1;
     constexpr bool KEEP = hess_keep<T, L, V>();
     const int tk = pick_tile<T, L, V>(ctx, MFIC_PASS_PAD_C2R_B, false);
@@ -754,31 +758,33 @@ static void launch_hess_b(mfic_ctx ctx, const cx<T>* xb, cx<T>* out, T kf) {
     const dim3 grid((unsigned)xcd_grid(ntiles), members);
     ProfScope prof(ctx, pass_name<T, L>("fft_c2rBh"), (double)cols * (members * N + 6 * L) * sizeof(cx<T>));
 #define CALL(K)                                                                                                \
-    hipLaunchKernelGGL((k_hess_b<T, L, K, V, KEEP>), grid, dim3(P * K), (pencil_lds<T, L, V>(K)), ctx->stream, \
+    hipLaunchKernelGGL((k_hess_b<T, W, L, K, V, KEEP>), grid, dim3(P * K), (pencil_lds<T, L, V>(K)), ctx->stream, \
                        LdAx1<T, true>{xb}, StAx1<T, false>{out}, cols, kf, tw);
     MFIC_TILE_SWITCH(P, CALL)
 #undef CALL
     MFIC_LAUNCH_CHECK();
 }
 
-template <typename T> void hessians_to_kbuf(mfic_ctx ctx, const void* f, size_t n, double L, void* xbuf, void* out) {
+template <typename T, typename W>
+void hessians_to_kbuf(mfic_ctx ctx, const void* f, size_t n, double L, void* xbuf, void* out) {
     const int np = 3 * (int)n / 2;
-    const T kf = (T)(2.0 * 3.14159265358979323846 / L), rfac = (T)std::pow(1.5, 1.5);
+    const W kf = (W)(2.0 * 3.14159265358979323846 / L), rfac = (W)std::pow(1.5, 1.5);
     const cx<T>* src = static_cast<const cx<T>*>(f);
-    cx<T>* xb = static_cast<cx<T>*>(xbuf);
-#define X(S)                                                                                                        \
-    case S:                                                                                                         \
-        if (plan_variant(ctx, S, MFIC_PASS_PAD_C2R_A, prec_of<T>()) == 1) launch_hess<T, S, alt_plan<S>()>(ctx, src, xb, kf, rfac); \
-        else launch_hess<T, S, 0>(ctx, src, xb, kf, rfac);                                                          \
-        if (plan_variant(ctx, S, MFIC_PASS_PAD_C2R_B, prec_of<T>()) == 1)                                           \
-            launch_hess_b<T, S, alt_plan<S>()>(ctx, xb, static_cast<cx<T>*>(out), kf);                              \
-        else launch_hess_b<T, S, 0>(ctx, xb, static_cast<cx<T>*>(out), kf);                                         \
+    cx<T>*xb = static_cast<cx<T>*>(xbuf), *ob = static_cast<cx<T>*>(out);
+#define X(S)                                                                                   \
+    case S:                                                                                    \
+        if (plan_variant(ctx, S, MFIC_PASS_PAD_C2R_A, prec_of<T>()) == 1)                      \
+            launch_hess<T, W, S, alt_plan<S>()>(ctx, src, xb, kf, rfac);                       \
+        else launch_hess<T, W, S, 0>(ctx, src, xb, kf, rfac);                                  \
+        if (plan_variant(ctx, S, MFIC_PASS_PAD_C2R_B, prec_of<T>()) == 1)                      \
+            launch_hess_b<T, W, S, alt_plan<S>()>(ctx, xb, ob, kf);                            \
+        else launch_hess_b<T, W, S, 0>(ctx, xb, ob, kf);                                       \
         break;
     MFIC_PADDED_SWITCH(np)
 #undef X
 }
 
-template <typename T, int L, int V> static void launch_hess_bt(mfic_ctx ctx, const cx<T>* in, cx<T>* zb, T kf) {
+template <typename T, int L, int V> static void launch_hess_bt(mfic_ctx ctx, const cx<T>* in, cx<T>* zb, double kf) {
     constexpr int P = Plan<L, V>::P, N = 2 * L / 3, kc = N / 2 + 1;
     const int tk = pick_tile<T, L, V>(ctx, MFIC_PASS_PAD_R2C_B, false);
     const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, PencilTw<T, L, V, 64>::KIND, prec_of<T>(), V));
@@ -793,7 +799,7 @@ template <typename T, int L, int V> static void launch_hess_bt(mfic_ctx ctx, con
     MFIC_LAUNCH_CHECK();
 }
 template <typename T, int L, int V>
-static void launch_hess_at(mfic_ctx ctx, const cx<T>* zb, const AdjointOut<T>& o, T kf) {
+static void launch_hess_at(mfic_ctx ctx, const cx<T>* zb, const AdjointOut<T>& o, double kf) {
     constexpr int P = Plan<L, V>::P, N = 2 * L / 3, kc = N / 2 + 1;
     const int tk = pick_tile<T, L, V>(ctx, MFIC_PASS_PAD_R2C_A, false);
     const cx<T>* tw = static_cast<const cx<T>*>(twiddles(ctx, L, PencilTw<T, L, V, 64>::KIND, prec_of<T>(), V));
@@ -812,7 +818,7 @@ template <typename T>
 void hessian_adjoint(mfic_ctx ctx, size_t n, double L, const void* prod, void* zbuf, const void* lam,
                      const double* tab, double g1, double volfac, void* out) {
     const int np = 3 * (int)n / 2;
-    const T kf = (T)(2.0 * 3.14159265358979323846 / L);
+    const double kf = 2.0 * 3.14159265358979323846 / L;
     const double rfac = std::sqrt((double)np * np * np) / std::sqrt((double)n * n * n);
     const double norm = 1.0 / std::sqrt((double)np * (double)np * (double)np);
     const AdjointOut<T> o{static_cast<cx<T>*>(out), static_cast<const cx<T>*>(lam), tab, g1, norm / rfac, volfac};
@@ -877,7 +883,7 @@ template <typename T> void truncate_repad(mfic_ctx ctx, size_t n, void* kbuf, in
 #define MFIC_PRUNED_T(MODE, T)                                                                                        \
     MODE template void operands_to_kbuf<T>(mfic_ctx, const OperandDesc*, int, size_t, const double*, void*);                \
     MODE template void r2c_from_kbuf<T>(mfic_ctx, size_t, double, void*, int, void* const*, int, double, bool);       \
-    MODE template void hessians_to_kbuf<T>(mfic_ctx, const void*, size_t, double, void*, void*);                      \
+    MODE template void hessians_to_kbuf<T, T>(mfic_ctx, const void*, size_t, double, void*, void*);                   \
     MODE template void hessian_adjoint<T>(mfic_ctx, size_t, double, const void*, void*, const void*, const double*,   \
                                           double, double, void*);                                                     \
     MODE template void truncate_repad<T>(mfic_ctx, size_t, void*, int);
@@ -887,9 +893,11 @@ MFIC_PRUNED_T(, double)
 #else
 MFIC_PRUNED_T(extern, double)
 
-void padded_hessians_to_kbuf(mfic_ctx ctx, int prec, const void* f, size_t n, double L, void* xbuf, void* out) {
-    if (prec == MFIC_F64) hessians_to_kbuf<double>(ctx, f, n, L, xbuf, out);
-    else hessians_to_kbuf<float>(ctx, f, n, L, xbuf, out);
+void padded_hessians_to_kbuf(mfic_ctx ctx, int prec, const void* f, size_t n, double L, void* xbuf, void* out,
+                             bool weights64) {
+    if (prec == MFIC_F64) hessians_to_kbuf<double, double>(ctx, f, n, L, xbuf, out);
+    else if (weights64) hessians_to_kbuf<float, double>(ctx, f, n, L, xbuf, out);
+    else hessians_to_kbuf<float, float>(ctx, f, n, L, xbuf, out);
 }
 
 void padded_hessian_adjoint(mfic_ctx ctx, int prec, size_t n, double L, const void* prod, void* zbuf, const void* lam,

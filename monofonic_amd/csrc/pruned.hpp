@@ -13,8 +13,10 @@ void padded_operands_to_kbuf(mfic_ctx ctx, int prec, const OperandDesc* o, int c
                              void* kbuf);
 // the six Hessians xx yy zz xy xz yz of an N-grid k-space field -> six
 // consecutive compact padded buffers (out) after the axis-0 and axis-1 c2r
-// passes; xbuf is scratch for three compact buffers
-void padded_hessians_to_kbuf(mfic_ctx ctx, int prec, const void* f, size_t n, double L, void* xbuf, void* out);
+// passes; xbuf is scratch for three compact buffers; weights64: gradient
+// factors in FP64 whatever the precision
+void padded_hessians_to_kbuf(mfic_ctx ctx, int prec, const void* f, size_t n, double L, void* xbuf, void* out,
+                             bool weights64 = false);
 // consecutive compact padded buffers of r2c'd rows of products (real space
 // along axes 0 and 1) -> the same buffers truncated to the source modes with
 // Nyquist planes zeroed and padded again, ready as inputs of a row pass: the
