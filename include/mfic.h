@@ -158,8 +158,7 @@ int mfic_fft_plan_count(int length);
 int mfic_fft_plan_info(int length, int variant, int *elems_per_thread, int radices[4]);
 /* select plan `variant` for one pass kind, length and precision on a
  * context; variant < 0 restores the default.  mfic_fft_get_plan reports
- * the current choice, mfic_fft_default_plan the built-in one. */
-int mfic_fft_default_plan(int length, int pass, int prec, int *variant);
+ * the current choice. */
 int mfic_fft_set_plan(mfic_ctx ctx, int length, int pass, int prec, int variant);
 int mfic_fft_get_plan(mfic_ctx ctx, int length, int pass, int prec, int *variant);
 

@@ -113,7 +113,6 @@ SIGNATURES = {
     "mfic_fft_get_tile": (C.c_int, [_P, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     "mfic_fft_plan_count": (C.c_int, [C.c_int]),
     "mfic_fft_plan_info": (C.c_int, [C.c_int, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
-    "mfic_fft_default_plan": (C.c_int, [C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int)]),
     "mfic_fft_set_plan": (C.c_int, [_P, C.c_int, C.c_int, C.c_int, C.c_int]),
     "mfic_fft_get_plan": (C.c_int, [_P, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int)]),
     "mfic_ngenic_seedtable": (C.c_int, [C.c_long, C.c_size_t, _P]),

@@ -152,16 +152,10 @@ def get_plan(ctx: Context, length: int, pass_kind: int, prec: int) -> int:
     return v.value
 
 
-def default_plan(length: int, pass_kind: int, prec: int) -> int:
-    """the plan a pass kind runs where none was selected"""
-    v = C.c_int()
-    L.call("mfic_fft_default_plan", length, pass_kind, prec, C.byref(v))
-    return v.value
-
-
 def chosen_plans(ctx: Context, n: int, prec: int) -> dict:
-    """{(length, pass kind): variant} of every non-default plan a box of
-    size n can use; set_plan of them on another context repeats the choice"""
+    """{(length, pass kind): variant} of every pass of a box of size n that
+    runs another plan than 0 (the 768-point FP32 truncation filters do so by
+    default)"""
     out = {}
     for length in (n, 3 * n // 2):
         for p in L.PASSES:
@@ -171,7 +165,7 @@ def chosen_plans(ctx: Context, n: int, prec: int) -> dict:
             elif plan_count(length) < 2:
                 continue
             v = get_plan(ctx, length, p, prec)
-            if v != default_plan(length, p, prec):
+            if v:
                 out[(length, p)] = v
     return out
 

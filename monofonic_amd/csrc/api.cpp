@@ -421,25 +421,17 @@ int mfic_fft_plan_info(int length, int variant, int* elems_per_thread, int radic
     });
 }
 
-static void check_plan_key(int length, int pass, int prec) {
+static void check_plan_key(mfic_ctx ctx, int length, int pass, int prec) {
+    MFIC_CHECK(ctx, MFIC_ERR_ARG, "null context");
     MFIC_CHECK(length > 0 && fft_length_supported(length), MFIC_ERR_SIZE, "unsupported FFT length");
     MFIC_CHECK(pass == MFIC_PASS_PENCILS || (pass >= MFIC_PASS_AX0_SHIFT && pass <= MFIC_PASS_FUSED_ROWS), MFIC_ERR_ARG,
                "pass must be one of mfic_fft_pass (row passes have one plan)");
     MFIC_CHECK(prec == MFIC_F32 || prec == MFIC_F64, MFIC_ERR_ARG, "bad precision");
 }
 
-int mfic_fft_default_plan(int length, int pass, int prec, int* variant) {
-    return guard([&] {
-        check_plan_key(length, pass, prec);
-        MFIC_CHECK(variant, MFIC_ERR_ARG, "null argument");
-        *variant = fft_default_plan(length, pass, prec);
-    });
-}
-
 int mfic_fft_set_plan(mfic_ctx ctx, int length, int pass, int prec, int variant) {
     return guard([&] {
-        MFIC_CHECK(ctx, MFIC_ERR_ARG, "null context");
-        check_plan_key(length, pass, prec);
+        check_plan_key(ctx, length, pass, prec);
         const auto key = std::make_tuple(length, pass, prec);
         if (variant < 0) { ctx->plans.erase(key); return; }
         if (pass == MFIC_PASS_FUSED_ROWS) {  // two forms at every padded length
@@ -455,8 +447,7 @@ int mfic_fft_set_plan(mfic_ctx ctx, int length, int pass, int prec, int variant)
 
 int mfic_fft_get_plan(mfic_ctx ctx, int length, int pass, int prec, int* variant) {
     return guard([&] {
-        MFIC_CHECK(ctx, MFIC_ERR_ARG, "null context");
-        check_plan_key(length, pass, prec);
+        check_plan_key(ctx, length, pass, prec);
         MFIC_CHECK(variant, MFIC_ERR_ARG, "null argument");
         *variant = plan_variant(ctx, length, pass, prec);
     });

@@ -140,7 +140,6 @@ const void* twiddles(mfic_ctx ctx, int L, int kind, int prec, int variant = 0);
 // the radix plan selected for a pass (mfic_fft_pass) of length L: the default
 // of the pass unless mfic_fft_set_plan chose one
 int plan_variant(mfic_ctx ctx, int L, int pass, int prec);
-int fft_default_plan(int L, int pass, int prec);
 // number of radix plans compiled for length L
 int fft_plan_count(int L);
 // elements per thread and radices of plan `variant` of length L
