@@ -153,9 +153,8 @@ def get_plan(ctx: Context, length: int, pass_kind: int, prec: int) -> int:
 
 
 def chosen_plans(ctx: Context, n: int, prec: int) -> dict:
-    """{(length, pass kind): variant} of every pass of a box of size n that
-    runs another plan than 0 (the 768-point FP32 truncation filters do so by
-    default)"""
+    """{(length, pass kind): variant} of every non-default plan a box of
+    size n can use; set_plan of them on another context repeats the choice"""
     out = {}
     for length in (n, 3 * n // 2):
         for p in L.PASSES:

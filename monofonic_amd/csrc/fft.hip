@@ -271,17 +271,13 @@ void fft_plan_info(int L, int variant, int* elems, int radices[4]) {
     }
 }
 
-// The truncation filters of 768-point FP32 pencils run on the 16-thread plan
-// by default: their two transforms are bound by barriers, which 256-thread
-// workgroups pay less for (four fields 4.94 ms against 5.55 on 32 threads; in
-// FP64, whose 48-element pencils spill, 10.3 against 9.4).
-static int default_plan(int L, int pass, int prec) {
-    return L == 768 && prec == MFIC_F32 && (pass == MFIC_PASS_TRUNC_AX0 || pass == MFIC_PASS_TRUNC_AX1) ? 1 : 0;
-}
-
+// Plan 0 unless the context selects another: with the twiddles in LDS it is the
+// better one of the 768-point truncation filters in both precisions (four
+// fields, axis 1 and 0: FP32 1.99 + 2.17 ms against 2.07 + 2.19 on the 16-thread
+// plan, FP64 4.87 + 4.75 against 5.29 + 5.27).
 int plan_variant(mfic_ctx ctx, int L, int pass, int prec) {
     const auto it = ctx->plans.find(std::make_tuple(L, pass, prec));
-    return it == ctx->plans.end() ? default_plan(L, pass, prec) : it->second;
+    return it == ctx->plans.end() ? 0 : it->second;
 }
 
 static std::vector<std::complex<long double>> make_table(int L, int kind, int variant) {

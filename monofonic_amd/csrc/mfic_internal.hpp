@@ -137,8 +137,8 @@ void require_device_memory(const void* p, const char* what);
 // shift phases exp(i pi m / L), m < 2L (kind 2, FP64); the inter-stage factors
 // follow radix plan `variant` of the length
 const void* twiddles(mfic_ctx ctx, int L, int kind, int prec, int variant = 0);
-// the radix plan selected for a pass (mfic_fft_pass) of length L: the default
-// of the pass unless mfic_fft_set_plan chose one
+// the radix plan selected for a pass (mfic_fft_pass) of length L (0 unless
+// mfic_fft_set_plan chose another)
 int plan_variant(mfic_ctx ctx, int L, int pass, int prec);
 // number of radix plans compiled for length L
 int fft_plan_count(int L);

@@ -9,6 +9,7 @@ import itertools
 
 import numpy as np
 import pytest
+import torch  # noqa: F401  before the library, whose HIP runtime is then torch's
 
 from monofonic_amd import F32, F64, Grid, _lib as L, lpt
 

@@ -6,6 +6,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import torch  # noqa: F401  before the library, whose HIP runtime is then torch's
 
 from monofonic_amd import F32, F64, Grid, _lib as L
 
