@@ -584,10 +584,11 @@ k_pencils_filter(LD ld, ST st, long ncols, const cx<T>* __restrict__ tw, int xcd
 
 // tile of a padded pass: the override of its own kind, else the override of
 // every strided pass of the length (kind 0), else 128-byte row segments (16
-// pencils in FP32, 8 in FP64).  Twice that for two plans: 16 threads of 24
-// elements per transform (384 points) in the passes with one output (`wide`),
-// whose workgroups are small, and 24 threads of 12 (288 points) in FP32, where
-// the Hessian passes take 106 + 277 us per 192^3 3LPT box against 121 + 327.
+// pencils in FP32, 8 in FP64).  Twice that at two lengths: 384 points in the
+// passes with one output (`wide`), whose workgroups are small (16 threads to a
+// transform, where the neighbouring lengths have 24 and 32), and 288 points in
+// FP32, where the Hessian passes take 106 + 277 us per 192^3 3LPT box against
+// 121 + 327.
 // Against the widest tile of 68 KB, which this is at 768 points: the two r2c
 // passes of four fields 84 -> 66 us at 192 points FP64, 42 -> 39 at 192 FP32.
 // Tiles below 4 run as 4.
@@ -595,7 +596,7 @@ template <typename T, int L, int V>
 static int pick_tile(mfic_ctx ctx, int pass, bool wide) {
     constexpr int P = Plan<L, V>::P;
     int tk = sizeof(T) == 8 ? 8 : 16;
-    if ((wide && V == 0 && P == 16 && Plan<L, V>::E >= 24) || (sizeof(T) == 4 && P == 24 && Plan<L, V>::E == 12)) tk *= 2;
+    if ((wide && L == 384) || (sizeof(T) == 4 && L == 288)) tk *= 2;
     const int prec = sizeof(T) == 8 ? MFIC_F64 : MFIC_F32;
     auto ov = ctx->tiles.find(std::make_tuple(L, pass, prec));
     if (ov == ctx->tiles.end()) ov = ctx->tiles.find(std::make_tuple(L, 0, prec));
