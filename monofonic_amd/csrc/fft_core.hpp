@@ -278,11 +278,13 @@ MFIC_SWZ(384, 0, 1, 3, 0, 4, 1)
 MFIC_SWZ(384, 1, 1, 4, 0, 6, 3)
 MFIC_SWZ(512, 0, 1, 4, 1, 5, 1)
 MFIC_SWZ(512, 1, 1, 5, 0, 6, 8)
-// plans of the paired fused passes: conflict-free both for 64-bit accesses
-// served 16 lanes at a time by 16 8-byte slots (the model that reproduces the
-// SQ_LDS_BANK_CONFLICT counts measured on MI355X) and for the 32-bit accesses of
-// FP32's split exchanges, 32 lanes at a time over 32 banks, with the transforms
-// of a wavefront a row pitch apart; 576 points on plan 0 within 9%
+// plans of the paired fused passes: searched to be conflict-free both for
+// 64-bit accesses served 16 lanes at a time by 16 8-byte slots (the model that
+// reproduces the SQ_LDS_BANK_CONFLICT counts of whole complex rows on MI355X)
+// and for the 32-bit accesses of FP32's split exchanges, 32 lanes at a time
+// over 32 banks, with the transforms of a wavefront a row pitch apart; 576
+// points on plan 0 within 9%.  Measured at 768 points, 16 inputs FP32: 1.9e7
+// conflict cycles of 1.1e9 active LDS cycles (4.7e6 with whole complex rows)
 MFIC_SWZ_V(768, 0, 3, 1, 3, 2, 5, 1)
 MFIC_SWZ_V(768, 1, 3, 1, 5, 0, 5, 4)
 MFIC_SWZ_V(768, 0, 2, 1, 4, 1, 6, 1)
@@ -433,8 +435,8 @@ __device__ __forceinline__ void fft_regs(cx<T>* v, int q, cx<T>* lds, MAP m, con
 // Pencil passes (TK neighbouring columns per workgroup) exchange real and
 // imaginary parts separately (SPLIT): with 16-column tiles of 768-point
 // pencils this lets three workgroups share a CU instead of one.
-// default LDS budget of a pencil tile: 128-byte row segments per pencil
-// position (16 complex FP32 columns) at 768 points, 32 at 512
+// LDS budget of a default tile of the two-output axis-0 pass, whose transforms
+// exchange in regions of their own: two workgroups a CU
 constexpr size_t PENCIL_LDS_CAP = 69632;
 template <typename T, int L, bool FWD, int V = 0, bool TWR = false>
 __device__ __forceinline__ void fft_pencil(cx<T>* v, int q, cx<T>* lds, LdsMap m, const cx<T>* __restrict__ tw) {
@@ -462,9 +464,10 @@ template <typename T, int L, int V, int THREADS> struct TwStage {
 // Twiddles of a pencil tile: in LDS for FP32, behind the exchange's `reals`
 // values.  A wavefront's 16-byte loads of them move 1 KB through the vector
 // cache whatever its lanes share, more than the data does; at 768 points FP32
-// the truncation passes go from 2.76 + 2.34 to 2.09 + 2.17 ms, at 384 the r2c
-// passes from 284 + 231 to 248 + 215 us.  FP64 tiles have half the lanes on
-// a factor and twice the LDS traffic: 288 points lose 3-9%, so they read memory.
+// the truncation passes go from 2.76 + 2.34 to 2.09 + 2.17 ms on the 16-thread
+// plan (1.99 + 2.17 on the default one), at 384 the r2c passes from 284 + 231 to
+// 248 + 215 us.  FP64 tiles have half the lanes on a factor and twice the LDS
+// traffic: 288 points lose 3-9%, so they read memory.
 template <typename T, int L, int V, int THREADS> struct PencilTw : TwStage<T, L, V, THREADS> {
     static constexpr bool LDS = sizeof(T) == 4;
     static constexpr int KIND = LDS ? 3 : 0;  // of the table

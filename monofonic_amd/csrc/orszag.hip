@@ -44,7 +44,7 @@ size_t ConvCore::kbuf_reals() const { return 2 * Np[0] * Np[1] * (N[2] / 2 + 1);
 // convolution.hh:495-518.  The padded real fields stay in the row pass's LDS
 // where they went through HBM, and a product of an operand with itself pads
 // and transforms it once: the seven products of the 2LPT source and one
-// convolve3 at 192^3 FP32 1.72 -> 1.11 ms.  Bound by the four strided passes
+// convolve3 at 192^3 FP32 1.72 -> 1.03 ms.  Bound by the four strided passes
 // (4.3-5.1 TB/s).
 void ConvCore::convolve2(const OperandDesc& a, const OperandDesc& b, void* out, int op, double coef, void* kbuf) const {
     const bool square = a.same(b);
