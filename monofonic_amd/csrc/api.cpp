@@ -40,11 +40,8 @@ void* ctx_scratch(mfic_ctx ctx, const std::string& key, size_t bytes) {
         if (s.captured && ctx->graphs > 0) ctx->retired.push_back(s.p);  // a graph's launches hold its address
         else if (s.p) MFIC_HIP(hipFree(s.p));
         s = mfic_scratch{};
-        hipError_t e = hipMalloc(&s.p, bytes);
-        if (e != hipSuccess) {
-            s.p = nullptr;
-            throw Error(MFIC_ERR_ALLOC, "scratch allocation of " + std::to_string(bytes) + " bytes failed");
-        }
+        s.p = device_alloc(bytes);
+        if (!s.p) throw Error(MFIC_ERR_ALLOC, "scratch allocation of " + std::to_string(bytes) + " bytes failed");
         s.bytes = bytes;
     }
     if (ctx->capturing) s.captured = true;
@@ -222,8 +219,8 @@ int mfic_grid_create(mfic_ctx ctx, const size_t n[3], const double L[3], int pre
         g->prec = prec;
         g->space = space;
         g->nreal = n[0] * n[1] * (n[2] + 2);
-        hipError_t e = hipMalloc(&g->d, g->bytes());
-        if (e != hipSuccess) {
+        g->d = device_alloc(g->bytes());
+        if (!g->d) {
             delete g;
             throw Error(MFIC_ERR_ALLOC, "device allocation of " + std::to_string(n[0] * n[1] * (n[2] + 2) * (prec ? 8 : 4)) + " bytes failed");
         }

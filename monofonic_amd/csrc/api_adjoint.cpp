@@ -153,11 +153,8 @@ int mfic_lpt2_create(mfic_ctx ctx, size_t n, double L, int prec, const mfic_cosm
         const double L3[3] = {L, L, L};
         p->core = std::make_unique<mfic::ConvCore>(ctx, n3, L3, prec);
         const size_t wsb = WS_BUFFERS * p->core->kbuf_reals() * p->core->esize();
-        if (hipMalloc(&p->ws, wsb) != hipSuccess) {
-            (void)hipGetLastError();
-            p->ws = nullptr;
-            throw Error(MFIC_ERR_ALLOC, "2LPT plan: workspace allocation of " + std::to_string(wsb) + " bytes failed");
-        }
+        p->ws = mfic::device_alloc(wsb);
+        MFIC_CHECK(p->ws, MFIC_ERR_ALLOC, "2LPT plan: workspace allocation of " + std::to_string(wsb) + " bytes failed");
         ++ctx->children;
         *out = p.release();
     });

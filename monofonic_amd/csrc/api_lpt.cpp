@@ -78,9 +78,8 @@ static OperandDesc to_desc(const mfic_operand* o, const ConvCore& c) {
 }
 
 static void* dmalloc(size_t bytes, const char* what) {
-    void* p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
-    if (e != hipSuccess) throw Error(MFIC_ERR_ALLOC, std::string("device allocation failed: ") + what);
+    void* p = device_alloc(bytes);
+    if (!p) throw Error(MFIC_ERR_ALLOC, std::string("device allocation failed: ") + what);
     return p;
 }
 

@@ -336,8 +336,12 @@ void* tk_upload(const mfic_cosmo_params& p, EhParams* eh) {
     }
     const std::vector<double> nodes = tk_spline_build(p.tk_k, p.tk_T, p.tk_n);
     void* d = nullptr;
-    if (hipMalloc(&d, nodes.size() * sizeof(double)) != hipSuccess) throw std::runtime_error("hipMalloc failed");
+    if (hipMalloc(&d, nodes.size() * sizeof(double)) != hipSuccess) {
+        (void)hipGetLastError();  // reported here, not by the next launch check
+        throw std::runtime_error("hipMalloc failed");
+    }
     if (hipMemcpy(d, nodes.data(), nodes.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
+        (void)hipGetLastError();
         (void)hipFree(d);
         throw std::runtime_error("hipMemcpy failed");
     }

@@ -25,11 +25,15 @@ struct Error : std::runtime_error {
 };
 void set_last_error(const std::string& msg);
 
+// a failing call also leaves its error with the thread, where the next launch
+// check would find it: it is taken from there when it is reported
 #define MFIC_HIP(call)                                                                      \
     do {                                                                                    \
         hipError_t e_ = (call);                                                             \
-        if (e_ != hipSuccess)                                                               \
+        if (e_ != hipSuccess) {                                                             \
+            (void)hipGetLastError();                                                        \
             throw ::mfic::Error(MFIC_ERR_HIP, std::string(#call) + ": " + hipGetErrorString(e_)); \
+        }                                                                                   \
     } while (0)
 #define MFIC_CHECK(cond, code, msg)                  \
     do {                                             \
@@ -119,6 +123,14 @@ class ProfScope {
     mfic_ctx ctx_;
     long idx_ = -1;
 };
+
+// device memory, or null (the caller reports it)
+inline void* device_alloc(size_t bytes) {
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
 
 // scratch buffer of at least `bytes`, keyed by name, owned by the context.  A
 // buffer that grows moves; the old one is freed unless a live graph uses it.
